@@ -44,16 +44,16 @@ struct Params {
     int segments;            // FP32 VJP: workgroups per tile, each over its own range of samples
     int base_tiles;          // tiles of one segment (total_tiles / segments)
     int segment_samples;     // samples per segment (a multiple of chunk_samples)
-    int slab_fallback;       // FP32 VJP: a chunk that overflows at the shortest length switches the workgroup to slab chunks
     int wt_x, wt_y, wt_per_view;  // wave tiles (8x8 pixels, or 64 rays) per view
     const double *panels;    // views x 12
     const double *ray_src;   // views x pixels x 3
     const double *ray_end;
     const double *poses;     // views x 12
     int *status;             // views
-    int brick_cap;           // FP64 LDS brick entries per workgroup (volume adjoint)
-    int slab_chunks;         // 1: the FP64 volume adjoint chunks by slabs of space, not by sample index
-    int chunk_samples;       // samples per lockstep chunk of the volume adjoint
+    int brick_cap;           // FP64 LDS brick entries per workgroup of the cell-Gauss volume adjoint
+    int walk_cap;            // FP64 LDS brick entries per workgroup of the midpoint volume adjoint
+    int slab_chunks;         // 1: index chunks would overflow even the larger brick often (silhouette-heavy plans)
+    int chunk_samples;       // unit of the sample segments
     int gauss_chunks;        // lockstep chunks per ray of the cell-Gauss volume adjoint
     const float *alpha;      // 2 x samples entries: alpha_k, then k + 0.5 (sample_table_entries)
     int volume_f64;          // 1: FP64 volume destination (increments unflushed, FP64 sampling unrounded)

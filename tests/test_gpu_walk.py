@@ -1,0 +1,86 @@
+"""The volume adjoint's cell walk on the GPU, at the sizes where it branches.
+
+``vol_walk_kernel`` forms each cell's corner sums in closed form from the
+cell's run of samples: singleton axes and half-cell borders, less than one
+sample per cell, thousands of samples per cell, axes beyond 2^18 grid samples
+(FP64 coordinates instead of biased ones), and slabs that fit no brick.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests import scenes
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+from .test_gpu_parity import NativeScene, _rel  # noqa: E402
+
+
+def _volume(grid, samples, precision, seed=0, views=3, rows=19, cols=21, rays=None):
+    panels = None if rays is not None else scenes.cone_panels(grid, views, rows, cols, sod=120.0, sdd=200.0, offset=0.3)
+    geometry = dict(rays=rays) if rays is not None else dict(panels=panels)
+    count = len(rays[0]) if rays is not None else views * rows * cols
+    seeds = np.random.default_rng(seed).uniform(-1.0, 1.0, count)
+    values = np.full(grid.voxels, 0.02, dtype=np.float32)
+    if precision == "float32":
+        seeds = seeds.astype(np.float32)
+    expected, _, _, _ = O.Scene(grid, samples, **geometry).vjp(
+        values, seeds, precision="fp32" if precision == "float32" else "fp64", pose=False)
+    actual, _, status = NativeScene(grid, samples, precision=precision, **geometry).vjp(values, seeds, pose_grad=False)
+    assert not any(status)
+    assert np.linalg.norm(expected) > 0
+    return actual, expected
+
+
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+@pytest.mark.parametrize("shape,samples", [((1, 26, 28), 97), ((24, 1, 28), 97), ((24, 26, 1), 97), ((2, 2, 2), 5),
+                                           ((24, 26, 28), 3), ((24, 26, 28), 31), ((3, 4, 5), 4001)])
+def test_cell_sums_match_the_per_sample_scatter(shape, samples, precision):
+    print(f"case walk {shape} S={samples} {precision}", flush=True)
+    grid = O.Grid(shape, (1.0, 0.9, 1.1), tuple(-0.5 * (n - 1) * h for n, h in zip(shape[::-1], (1.0, 0.9, 1.1))))
+    actual, expected = _volume(grid, samples, precision)
+    # FP32: the oracle rounds each sample's position, |p| <= 200 mm at 2^-24
+    # (1.2e-5 voxel), and increments to FP32; FP64: FP32-rounded increments
+    # and one FP32 rounding of the result
+    assert _rel(actual, expected) <= (1e-5 if precision == "float32" else 1e-7)
+
+
+@pytest.mark.parametrize("cap", ["512", "8192"])
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+def test_slabs_that_fit_no_brick_use_device_atomics(cap, precision, monkeypatch):
+    print(f"case walk cap={cap} {precision}", flush=True)
+    monkeypatch.setenv("DPT_AMD_BRICK_CAP", cap)
+    grid = O.Grid((40, 44, 48), (1.0, 1.0, 1.0), (-23.5, -21.5, -19.5))
+    actual, expected = _volume(grid, 61, precision, rows=16, cols=16)  # about 4 voxels between pixels
+    assert _rel(actual, expected) <= (1e-5 if precision == "float32" else 1e-7)
+
+
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+def test_axes_beyond_the_biased_coordinates(precision):
+    """2^18 + 40 grid samples along x: FP32 sampling resolves positions to
+    2^18 * 2^-24 = 1/64 voxel, so its gradient is compared through its total
+    (each ray's weights sum to one per sample); FP64 element by element."""
+    print(f"case walk wide {precision}", flush=True)
+    n = (1 << 18) + 40
+    grid = O.Grid((3, 2, n), (1.0, 1.0, 1.0))
+    src = np.array([[n - 80.25, 0.5, 1.0], [n - 90.0, -0.2, 0.4], [-3.0, 0.4, 1.1]])
+    end = np.array([[n + 30.0, 0.6, 1.2], [n - 20.0, 1.2, 1.7], [50.0, 0.7, 0.9]])
+    actual, expected = _volume(grid, 257, precision, rays=(src, end))
+    if precision == "float64":
+        assert _rel(actual, expected) <= 1e-7
+    else:
+        assert abs(actual.sum(dtype=np.float64) / expected.sum(dtype=np.float64) - 1.0) <= 1e-5
+        assert _rel(actual, expected) <= 5e-2
+
+
+def test_more_samples_than_the_float_counter_holds():
+    print("case walk S=5e6", flush=True)
+    grid = O.Grid((3, 3, 3), (1.0, 1.0, 1.0))
+    rays = (np.array([[-4.0, 0.3, 0.9]]), np.array([[7.0, 1.4, 1.6]]))
+    actual, expected = _volume(grid, 5_000_000, "float32", rays=rays)
+    assert _rel(actual, expected) <= 1e-5
