@@ -30,6 +30,7 @@ constexpr int kRayTangent = 8;
 struct Params {
     int nx, ny, nz;
     int ix, iy;              // row / slab counts of the gather index: (nx, ny) linear, cell counts for cells
+    int qz;                  // quads per plane of the quad layout (0 for a singleton z axis)
     int sx, sy, sz;          // corner strides: 1, nx, nx*ny, or 0 for singleton axes
     float hx, hy, hz;        // n - 0.5 (upper support bound)
     float cx, cy, cz;        // n - 1 (upper clamp)
@@ -55,7 +56,7 @@ struct Params {
     int slab_chunks;         // 1: index chunks would overflow even the larger brick often (silhouette-heavy plans)
     int chunk_samples;       // unit of the sample segments
     int gauss_chunks;        // lockstep chunks per ray of the cell-Gauss volume adjoint
-    const float *alpha;      // 2 x samples entries: alpha_k, then k + 0.5 (sample_table_entries)
+    const float *alpha;      // 3 x samples entries: alpha_k, k + 0.5, 1 - alpha_k (sample_table_entries)
     int volume_f64;          // 1: FP64 volume destination (increments unflushed, FP64 sampling unrounded)
 };
 
@@ -66,12 +67,14 @@ struct Params {
 //     (kernels/projection_fp32.py:455-458; IEEE binary32 division, identical
 //     to the device's correctly rounded division);
 //   c_k = k + 0.5, the sample centre (kernels/projection_fp32.py:116-119;
-//     exact in FP32 for k < 2^23).
-inline size_t sample_table_entries(int samples) { return 2 * (size_t)samples; }
+//     exact in FP32 for k < 2^23);
+//   RN(1 - alpha_k).
+inline size_t sample_table_entries(int samples) { return 3 * (size_t)samples; }
 inline void fill_alpha_table(float *out, int samples) {
     for (int k = 0; k < samples; ++k) {
         out[k] = ((float)k + 0.5f) / (float)samples;
         out[samples + k] = (float)k + 0.5f;
+        out[2 * (size_t)samples + k] = 1.0f - out[k];
     }
 }
 
@@ -80,6 +83,10 @@ inline void fill_alpha_table(float *out, int samples) {
 __device__ __forceinline__ float sample_alpha(const Params &P, int k) {
     typedef const float __attribute__((address_space(4))) *constant_t;
     return ((constant_t)P.alpha)[k];
+}
+__device__ __forceinline__ float sample_beta(const Params &P, int k) {
+    typedef const float __attribute__((address_space(4))) *constant_t;
+    return ((constant_t)P.alpha)[2 * (size_t)P.samples + k];
 }
 __device__ __forceinline__ float sample_centre(const Params &P, int k) {
     typedef const float __attribute__((address_space(4))) *constant_t;
@@ -425,6 +432,87 @@ __device__ __forceinline__ bool cell32(const Params &P, float p0, float p1, floa
     return true;
 }
 
+// Minimum over the wave; every lane must be active.
+__device__ __forceinline__ int wave_min(int v) {
+    // rows of 16, then across rows: lane 63 holds the minimum of the wave
+    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// A point in [0, n - 1) on every axis, where cell32_inside's clamps and caps
+// are identities and its slopes are one: the same cell and fractions from 13
+// VALU instructions instead of 32 (fract(p) = p - floor(p) is exact for
+// p >= 0).
+__device__ __forceinline__ void cell32_interior(const Params &P, float p0, float p1, float p2, Cell32 &c) {
+    c.lx = (int)p0;
+    c.ly = (int)p1;
+    c.lz = (int)p2;
+    c.fx = __builtin_amdgcn_fractf(p0);
+    c.fy = __builtin_amdgcn_fractf(p1);
+    c.fz = __builtin_amdgcn_fractf(p2);
+    c.slx = c.sly = c.slz = 1.0f;
+    c.base = (int)(__umul24(__umul24((unsigned)c.lz, (unsigned)P.iy) + (unsigned)c.ly, (unsigned)P.ix) +
+                   (unsigned)c.lx);
+}
+
+__device__ __forceinline__ bool interior32(const Params &P, float p0, float p1, float p2) {
+    return p0 >= 0.0f && p1 >= 0.0f && p2 >= 0.0f && p0 < P.cx && p1 < P.cy && p2 < P.cz;
+}
+
+// Samples [ka, kb) of [k0, k1) that are interior points for every active lane
+// of the wave (uniform; empty when there are none).  Estimated from the rays'
+// crossings of the planes 0 and n - 1 with a margin of two samples, then both
+// ends are tested as sampled: coordinates are monotone in the sample index, so
+// the samples between two interior ones are interior.
+__device__ __forceinline__ void interior_span(const Params &P, const float *o, const float *d, float lower, float step,
+                                              int k0, int k1, int &ka, int &kb) {
+    const float top[3] = {P.cx, P.cy, P.cz};
+    float enter = lower, leave = 3e38f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float inverse = __builtin_amdgcn_rcpf(d[a]);
+        const float u = (0.0f - o[a]) * inverse, v = (top[a] - o[a]) * inverse;
+        enter = fmaxf(enter, fminf(u, v));
+        leave = fminf(leave, fmaxf(u, v));
+    }
+    const float per = __builtin_amdgcn_rcpf(step);
+    const float lo = fminf(fmaxf(ceilf((enter - lower) * per) + 2.0f, (float)k0), (float)k1);
+    const float hi = fminf(fmaxf(floorf((leave - lower) * per) - 2.0f, (float)k0), (float)k1);
+    // the latest entry and the earliest exit of the active lanes, by bisection
+    // (cross-lane reductions would read lanes that this branch masks)
+    int below = k0, above = k1;
+    while (below < above) {
+        const int m = (below + above) >> 1;
+        if (__builtin_amdgcn_ballot_w64((int)lo > m) != 0)
+            below = m + 1;
+        else
+            above = m;
+    }
+    ka = below;
+    below = k0;
+    above = k1;
+    while (below < above) {
+        const int m = (below + above + 1) >> 1;
+        if (__builtin_amdgcn_ballot_w64((int)hi < m) != 0)
+            above = m - 1;
+        else
+            below = m;
+    }
+    kb = below;
+    if (kb > ka) {
+        const float a = fmaf(sample_centre(P, ka), step, lower), b = fmaf(sample_centre(P, kb - 1), step, lower);
+        const bool ok = interior32(P, fmaf(a, d[0], o[0]), fmaf(a, d[1], o[1]), fmaf(a, d[2], o[2])) &&
+                        interior32(P, fmaf(b, d[0], o[0]), fmaf(b, d[1], o[1]), fmaf(b, d[2], o[2]));
+        if (__builtin_amdgcn_ballot_w64(!ok) != 0) kb = ka;
+    }
+    if (kb <= ka) ka = kb = k1;
+}
+
 // corner k value offsets: bit0 x, bit1 y, bit2 z (kernels/projection.py:217-222;
 // lower <= n-2 so only singleton axes clamp, which a zero stride reproduces).
 __device__ __forceinline__ int corner_offset(const Params &P, int k) {
@@ -487,6 +575,7 @@ __device__ __forceinline__ float load_global<__half>(global_const<__half> *f, in
 constexpr int kLayoutScalar = 0;  // linear field, eight scalar loads (nx == 1)
 constexpr int kLayoutPair = 1;    // linear field, x-adjacent pairs (nx > 1)
 constexpr int kLayoutCells = 2;   // cell layout (DPT_STORE_CELLS): one cell per gather
+constexpr int kLayoutQuads = 3;   // quad layout (a plan's own FP32 copy): the cell's two z faces, 4 corners each
 
 struct __attribute__((aligned(16))) Quad {
     uint32_t x, y, z, w;
@@ -495,7 +584,21 @@ struct __attribute__((aligned(16))) Quad {
 template <typename T, int LAYOUT>
 __device__ __forceinline__ void load8(const Params &P, const T *field_any, int base, float *v) {
     global_const<T> *field = (global_const<T> *)field_any;
-    if constexpr (LAYOUT == kLayoutCells && std::is_same<T, float>::value) {
+    if constexpr (LAYOUT == kLayoutQuads) {
+        // 16-byte quads of planes z and z + 1
+        global_const<Quad> *q = reinterpret_cast<global_const<Quad> *>(field) + (size_t)(unsigned)base;
+        global_const<Quad> *r = reinterpret_cast<global_const<Quad> *>(field) + (size_t)(unsigned)(base + P.qz);
+        const Quad a = {q->x, q->y, q->z, q->w};
+        const Quad b = {r->x, r->y, r->z, r->w};
+        v[0] = __uint_as_float(a.x);
+        v[1] = __uint_as_float(a.y);
+        v[2] = __uint_as_float(a.z);
+        v[3] = __uint_as_float(a.w);
+        v[4] = __uint_as_float(b.x);
+        v[5] = __uint_as_float(b.y);
+        v[6] = __uint_as_float(b.z);
+        v[7] = __uint_as_float(b.w);
+    } else if constexpr (LAYOUT == kLayoutCells && std::is_same<T, float>::value) {
         // 32-byte cell: corners 0-3 then 4-7, two 16-byte loads
         global_const<Quad> *q = reinterpret_cast<global_const<Quad> *>(field) + 2 * (size_t)base;
         const Quad a = {q[0].x, q[0].y, q[0].z, q[0].w};

@@ -15,8 +15,8 @@
 // workgroup of 256 lanes owns one 16x16 detector tile of one view, or 8x8
 // tiles of four consecutive views (one wave64 each); workgroup ids are
 // remapped so each XCD walks a contiguous range of tiles.  Corners are
-// gathered from the linear field (x-adjacent pairs) or from a cell-layout copy
-// (8 corners per cell, one or two 16-byte loads).  Pose cotangents are
+// gathered from the linear field (x-adjacent pairs) or from a copy (FP32: quads
+// of 4 corners per plane, 16-bit: cells of 8; two or one 16-byte loads).  Pose cotangents are
 // reduced per ray in FP64, across the wave with shuffles, then across tiles in
 // a fixed-order FP64 pass.  Volume cotangents are a launch of their own: a lane
 // steps from cell to cell along its ray, adds each cell's eight corner sums to
@@ -99,17 +99,22 @@ __global__ __launch_bounds__(kBlock) void forward32_kernel(Params P, const T *__
         bad = !finite_span(o, d, iv.lower, step, 0, P.samples);
         float v[8];
         int cur = -1;
-        auto walk = [&](auto check) {
-            constexpr bool CHECK = decltype(check)::value;
-            for (int k = 0; k < P.samples; ++k) {
+        auto walk = [&](auto interior, int k0, int k1, bool checked) {
+            constexpr bool INTERIOR = decltype(interior)::value;
+            for (int k = k0; k < k1; ++k) {
                 if constexpr (COMPENSATED) {
                     if (k > 0 && (k % kFoldBlock) == 0) total.fold();
                 }
-                float pos;
+                const float pos = fmaf(sample_centre(P, k), step, iv.lower);
+                const float p0 = fmaf(pos, d[0], o[0]);
+                const float p1 = fmaf(pos, d[1], o[1]);
+                const float p2 = fmaf(pos, d[2], o[2]);
                 Cell32 c;
-                sample_at<CHECK>(P, o, d, iv.lower, step, k, pos, c);
-                if constexpr (CHECK) {
-                    if (c.base < 0) continue;
+                if constexpr (INTERIOR) {
+                    cell32_interior(P, p0, p1, p2, c);
+                } else {
+                    if (checked && !inside32(P, p0, p1, p2)) continue;
+                    cell32_inside(P, p0, p1, p2, c);
                 }
                 if (c.base != cur) {
                     load8<T, LAYOUT>(P, field, c.base, v);
@@ -172,12 +177,16 @@ __global__ __launch_bounds__(kBlock) void forward32_kernel(Params P, const T *__
 #pragma unroll
             for (int j = 0; j < kPipeDepth; ++j)
                 if (k0 + j < last) consume(j);  // uniform
-        } else if (__builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, 0, P.samples)) == 0) {
-            // per-sample support tests only for waves with a ray whose end
-            // samples leave the support
-            walk(std::false_type{});
         } else {
-            walk(std::true_type{});
+            // per-sample support tests only for waves with a ray whose end
+            // samples leave the support; clamps only outside the samples that
+            // are interior points for the whole wave
+            const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, 0, P.samples)) != 0;
+            int ka, kb;
+            interior_span(P, o, d, iv.lower, step, 0, P.samples, ka, kb);
+            walk(std::false_type{}, 0, ka, checked);
+            walk(std::true_type{}, ka, kb, false);
+            walk(std::false_type{}, kb, P.samples, checked);
         }
         if (bad) flag(P, view, DPT_STATUS_RANGE);
         result = total.value() * (len * step);
@@ -417,17 +426,6 @@ int choose_brick_cap(const Params &P, const double *panels, int *slab_chunks) {
     return measured > 0 && 4 * rescued >= measured ? 2 * kBrickCapDefault : kBrickCapDefault;
 }
 
-__device__ __forceinline__ int wave_min(int v) {
-    // rows of 16, then across rows: lane 63 holds the minimum of the wave
-    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x111, 0xf, 0xf, false));  // row_shr:1
-    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x112, 0xf, 0xf, false));  // row_shr:2
-    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x114, 0xf, 0xf, false));  // row_shr:4
-    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x118, 0xf, 0xf, false));  // row_shr:8
-    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-    v = min(v, __builtin_amdgcn_update_dpp(INT_MAX, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-    return __builtin_amdgcn_readlane(v, 63);
-}
-
 // Bound one chunk's cells over the workgroup and, when the box fits the LDS
 // brick, describe it.  lo / nhi: this lane's lower cell corner minimum and
 // negated maximum over its chunk samples (INT_MAX when it has none).  Every
@@ -651,62 +649,75 @@ __global__ __launch_bounds__(kBlock) void vjp32_kernel(Params P, const T *__rest
         } else {
             float v[8];
             int cur = -1;
-            // per-sample support tests only for waves with a ray whose ends
-            // leave the support (uniform over the wave)
-            const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, first, last)) != 0;
-            for (int k = first; k < last; ++k) {
-                if constexpr (COMPENSATED) {
-                    if (k > first && ((k - first) % kFoldBlock) == 0) {
-                        mean.fold();
-                        dor0.fold();
-                        dor1.fold();
-                        dor2.fold();
-                        dd0.fold();
-                        dd1.fold();
-                        dd2.fold();
-                        shl.fold();
-                        shu.fold();
+            auto walk = [&](auto interior, int k0, int k1, bool checked) {
+                constexpr bool INTERIOR = decltype(interior)::value;
+                for (int k = k0; k < k1; ++k) {
+                    if constexpr (COMPENSATED) {
+                        if (k > first && ((k - first) % kFoldBlock) == 0) {
+                            mean.fold();
+                            dor0.fold();
+                            dor1.fold();
+                            dor2.fold();
+                            dd0.fold();
+                            dd1.fold();
+                            dd2.fold();
+                            shl.fold();
+                            shu.fold();
+                        }
                     }
+                    const float pos = fmaf(sample_centre(P, k), step, iv.lower);
+                    const float p0 = fmaf(pos, d[0], o[0]);
+                    const float p1 = fmaf(pos, d[1], o[1]);
+                    const float p2 = fmaf(pos, d[2], o[2]);
+                    Cell32 c;
+                    float live = 1.0f;
+                    if constexpr (INTERIOR) {
+                        cell32_interior(P, p0, p1, p2, c);
+                    } else {
+                        cell32_inside(P, p0, p1, p2, c);
+                        if (checked) {  // outside samples add nothing
+                            const bool inside = inside32(P, p0, p1, p2);
+                            c.fx = inside ? c.fx : 0.0f;
+                            c.fy = inside ? c.fy : 0.0f;
+                            c.fz = inside ? c.fz : 0.0f;
+                            c.slx = inside ? c.slx : 0.0f;
+                            c.sly = inside ? c.sly : 0.0f;
+                            c.slz = inside ? c.slz : 0.0f;
+                            live = inside ? 1.0f : 0.0f;
+                        }
+                    }
+                    if (c.base != cur) {
+                        load8<T, LAYOUT>(P, field, c.base, v);
+                        cur = c.base;
+                    }
+                    float wt[8], g[3];
+                    weights32(c, wt);
+                    // an outside sample's slopes are zero (above); its value is zeroed here
+                    const float value = INTERIOR ? interpolate32(wt, v) : interpolate32(wt, v) * live;
+                    slopes32(c, v, g);
+                    mean.add(value);
+                    dor0.add(g[0]);
+                    dor1.add(g[1]);
+                    dor2.add(g[2]);
+                    // contracted by the reference's code generator (fuse_fp)
+                    dd0.fma_add(pos, g[0]);
+                    dd1.fma_add(pos, g[1]);
+                    dd2.fma_add(pos, g[2]);
+                    const float along = fmaf(g[2], d[2], fmaf(g[1], d[1], g[0] * d[0]));
+                    shl.fma_add(sample_beta(P, k), along);
+                    shu.fma_add(sample_alpha(P, k), along);
                 }
-                const float pos = fmaf(sample_centre(P, k), step, iv.lower);
-                const float p0 = fmaf(pos, d[0], o[0]);
-                const float p1 = fmaf(pos, d[1], o[1]);
-                const float p2 = fmaf(pos, d[2], o[2]);
-                Cell32 c;
-                cell32_inside(P, p0, p1, p2, c);
-                float live = 1.0f;
-                if (checked) {  // outside samples add nothing
-                    const bool inside = inside32(P, p0, p1, p2);
-                    c.fx = inside ? c.fx : 0.0f;
-                    c.fy = inside ? c.fy : 0.0f;
-                    c.fz = inside ? c.fz : 0.0f;
-                    c.slx = inside ? c.slx : 0.0f;
-                    c.sly = inside ? c.sly : 0.0f;
-                    c.slz = inside ? c.slz : 0.0f;
-                    live = inside ? 1.0f : 0.0f;
-                }
-                if (c.base != cur) {
-                    load8<T, LAYOUT>(P, field, c.base, v);
-                    cur = c.base;
-                }
-                float wt[8], g[3];
-                weights32(c, wt);
-                // an outside sample's slopes are zero (above); its value is zeroed here
-                const float value = interpolate32(wt, v) * live;
-                slopes32(c, v, g);
-                mean.add(value);
-                dor0.add(g[0]);
-                dor1.add(g[1]);
-                dor2.add(g[2]);
-                // contracted by the reference's code generator (fuse_fp)
-                dd0.fma_add(pos, g[0]);
-                dd1.fma_add(pos, g[1]);
-                dd2.fma_add(pos, g[2]);
-                const float alpha = sample_alpha(P, k);
-                const float along = fmaf(g[2], d[2], fmaf(g[1], d[1], g[0] * d[0]));
-                shl.fma_add(1.0f - alpha, along);
-                shu.fma_add(alpha, along);
-            }
+            };
+            // per-sample support tests only for waves with a ray whose end
+            // samples leave the support (uniform over the wave); clamps and
+            // slope flags only outside the samples that are interior points
+            // for the whole wave (full scan: 86.9 -> 75.9 ms)
+            const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, first, last)) != 0;
+            int ka, kb;
+            interior_span(P, o, d, iv.lower, step, first, last, ka, kb);
+            walk(std::false_type{}, first, ka, checked);
+            walk(std::true_type{}, ka, kb, false);
+            walk(std::false_type{}, kb, last, checked);
         }
     }
     double gradient[kMaxComponents];
@@ -1976,6 +1987,22 @@ __global__ __launch_bounds__(kBlock) void cells_kernel(const E *__restrict__ src
     }
 }
 
+// Linear FP32 field -> quad layout, one lane per (i, j, plane): corners (i, j),
+// (i+1, j), (i, j+1), (i+1, j+1) of the plane, +1 neighbours clamped as in the
+// cell layout.
+__global__ __launch_bounds__(kBlock) void quads_kernel(const uint32_t *__restrict__ src, Quad *__restrict__ dst, int nx,
+                                                       int ny, int mx, int my, int64_t quads) {
+    for (int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x; c < quads; c += (int64_t)gridDim.x * kBlock) {
+        const int i = (int)(c % mx);
+        const int64_t r = c / mx;
+        const int j = (int)(r % my);
+        const int64_t k = r / my;
+        const int i1 = min(i + 1, nx - 1), j1 = min(j + 1, ny - 1);
+        const int64_t a = (k * ny + j) * nx, b = (k * ny + j1) * nx;
+        dst[c] = Quad{src[a + i], src[a + i1], src[b + i], src[b + i1]};
+    }
+}
+
 // Count rays whose FP32 clipped interval is non-empty (effective samples =
 // count * samples); same setup arithmetic as the forward kernel.
 __global__ __launch_bounds__(kBlock) void count_hits_kernel(Params P, unsigned long long *count) {
@@ -2056,10 +2083,9 @@ struct dpt_plan {
     float *d_alpha = nullptr;
     unsigned long long *d_count = nullptr;
     bool cell_gauss = false;  // FP64 exact cell-Gauss integration instead of midpoints
-    bool cells = false;       // FP32 sampling gathers from the cell-layout copy
+    bool cells = false;       // FP32 sampling gathers from the plan's copy: quads (FP32) or cells (16-bit)
     int mx = 1, my = 1;       // cells along x and y
-    int64_t cell_count = 0;
-    void *d_cells = nullptr;  // 8 * cell_count elements of the storage type
+    void *d_copy = nullptr;   // the gather copy
     int vjp_vb = 1;          // views per workgroup of the VJP launches
     int forward_vb = 1;      // views per workgroup of the forward launch
     bool timing = false;
@@ -2281,12 +2307,21 @@ Params launch_params(const dpt_plan *p, const double *poses) {
 
 unsigned tile_grid(const Params &P) { return (unsigned)(P.chunk * kXcds); }
 
-// Launch parameters of a gather from the plan's cell-layout copy.
-Params cells_params(const dpt_plan *p, Params P) {
+// Launch parameters of a gather from the plan's copy (quads or cells).
+Params copy_params(const dpt_plan *p, Params P) {
     P.ix = p->mx;
     P.iy = p->my;
+    P.qz = P.nz > 1 ? p->mx * p->my : 0;
     return P;
 }
+
+// Layout of the plan's copy.  FP32: quads, 16 bytes a load, neighbouring
+// lanes' quads adjacent, half the copy of 32-byte cells (full scan, against
+// cells: forward 57.2 -> 53.8 ms, pose VJP 75.9 -> 72.2, the copy 0.15 -> 0.06).
+// 16-bit: cells, whose one 16-byte load halves the load instructions (24
+// views of 256^2 over 256^3 in bfloat16: forward 2.0 ms, with quads 3.4).
+template <typename T>
+constexpr int kGatherCopy = std::is_same<T, float>::value ? kLayoutQuads : kLayoutCells;
 
 template <typename T>
 int launch_forward(dpt_plan *p, const Params &P, const void *field, void *out, bool cells, hipStream_t s) {
@@ -2298,8 +2333,8 @@ int launch_forward(dpt_plan *p, const Params &P, const void *field, void *out, b
         if constexpr (!HALF) {
             if (small_launch(P)) {
                 if (cells)
-                    hipLaunchKernelGGL((forward32_kernel<T, false, kLayoutCells, true>), grid, block, 0, s,
-                                       cells_params(p, P), static_cast<const T *>(p->d_cells), o);
+                    hipLaunchKernelGGL((forward32_kernel<T, false, kGatherCopy<T>, true>), grid, block, 0, s,
+                                       copy_params(p, P), static_cast<const T *>(p->d_copy), o);
                 else if (P.nx > 1)
                     hipLaunchKernelGGL((forward32_kernel<T, false, kLayoutPair, true>), grid, block, 0, s, P, f, o);
                 else
@@ -2310,8 +2345,8 @@ int launch_forward(dpt_plan *p, const Params &P, const void *field, void *out, b
             }
         }
         if (cells)
-            hipLaunchKernelGGL((forward32_kernel<T, HALF, kLayoutCells>), grid, block, 0, s, cells_params(p, P),
-                               static_cast<const T *>(p->d_cells), o);
+            hipLaunchKernelGGL((forward32_kernel<T, HALF, kGatherCopy<T>>), grid, block, 0, s, copy_params(p, P),
+                               static_cast<const T *>(p->d_copy), o);
         else if (P.nx > 1)
             hipLaunchKernelGGL((forward32_kernel<T, HALF, kLayoutPair>), grid, block, 0, s, P, f, o);
         else
@@ -2356,7 +2391,7 @@ int launch_vjp_c(dpt_plan *p, const Params &P, const void *field, const void *se
     if (p->arithmetic == DPT_ARITH_FP32) {
         const float *sd = static_cast<const float *>(seeds);
         if (cells && P.nx > 1)
-            launch_vjp32<T, C, kLayoutCells>(p, cells_params(p, P), static_cast<const T *>(p->d_cells), sd, pipe, s);
+            launch_vjp32<T, C, kGatherCopy<T>>(p, copy_params(p, P), static_cast<const T *>(p->d_copy), sd, pipe, s);
         else if (P.nx > 1)
             launch_vjp32<T, C, kLayoutPair>(p, P, f, sd, pipe, s);
         else
@@ -2423,8 +2458,15 @@ int launch_cells(const void *src, void *dst, int nx, int ny, int nz, int storage
     return DPT_OK;
 }
 
-int refresh_cells(dpt_plan *p, const void *field, hipStream_t s) {
-    return launch_cells(field, p->d_cells, p->base.nx, p->base.ny, p->base.nz, p->storage, s);
+// Rebuild the plan's gather copy of the field.
+int refresh_copy(dpt_plan *p, const void *field, hipStream_t s) {
+    const Params &P = p->base;
+    if (p->storage != DPT_STORE_F32) return launch_cells(field, p->d_copy, P.nx, P.ny, P.nz, p->storage, s);
+    const int64_t quads = (int64_t)p->mx * p->my * P.nz;
+    hipLaunchKernelGGL(quads_kernel, dim3(grid_blocks(quads)), dim3(kBlock), 0, s, static_cast<const uint32_t *>(field),
+                       static_cast<Quad *>(p->d_copy), P.nx, P.ny, p->mx, p->my, quads);
+    HIP_TRY(hipGetLastError());
+    return DPT_OK;
 }
 
 void timer_begin(dpt_plan *p, int kind, hipStream_t s) {
@@ -2455,7 +2497,7 @@ int dpt_plan_destroy(dpt_plan *p) {
     (void)hipFree(p->d_partials);
     (void)hipFree(p->d_acc);
     (void)hipFree(p->d_alpha);
-    (void)hipFree(p->d_cells);
+    (void)hipFree(p->d_copy);
     (void)hipFree(p->d_count);
     (void)hipFree(p->d_gather_rays);
     (void)hipFree(p->d_gather_views);
@@ -2599,7 +2641,7 @@ int plan_create(const dpt_grid_desc *grid, int32_t views, int32_t rows, int32_t 
     p->cells = p->cells && arithmetic == DPT_ARITH_FP32;
     p->mx = grid->nx > 1 ? grid->nx - 1 : 1;
     p->my = grid->ny > 1 ? grid->ny - 1 : 1;
-    p->cell_count = (int64_t)p->mx * p->my * (grid->nz > 1 ? grid->nz - 1 : 1);
+    const int64_t planes = (int64_t)p->mx * p->my;
 
     auto cleanup = [&](int code, const std::string &msg) {
         dpt_plan_destroy(p);
@@ -2648,7 +2690,8 @@ int plan_create(const dpt_grid_desc *grid, int32_t views, int32_t rows, int32_t 
         return cleanup(DPT_E_MEMORY, "pinned status allocation failed");
     if (needs & DPT_POSE) ALLOC(p->d_partials, sizeof(double) * kMaxComponents * (size_t)P.wt_per_view * views);
     if (needs & DPT_VOLUME) ALLOC(p->d_acc, sizeof(double) * (size_t)voxels);
-    if (p->cells) ALLOC(p->d_cells, (storage == DPT_STORE_F32 ? 4 : 2) * 8 * (size_t)p->cell_count);
+    if (p->cells) ALLOC(p->d_copy, storage == DPT_STORE_F32 ? 16 * (size_t)(planes * grid->nz)
+                                                        : 16 * (size_t)(planes * std::max(grid->nz - 1, 1)));
     ALLOC(p->d_count, sizeof(unsigned long long));
     ALLOC(p->d_alpha, sizeof(float) * sample_table_entries(samples));
     {
@@ -2707,7 +2750,7 @@ int dpt_forward(dpt_plan *p, const void *field, const double *poses, void *out, 
     hipLaunchKernelGGL(check_poses_kernel, dim3((P.views + 63) / 64), dim3(64), 0, s, poses, P.views, p->d_status);
     HIP_TRY(hipGetLastError());
     if (p->cells) {
-        const int rc = refresh_cells(p, field, s);
+        const int rc = refresh_copy(p, field, s);
         if (rc != DPT_OK) return rc;
     }
     timer_begin(p, 0, s);
@@ -2790,7 +2833,7 @@ int dpt_vjp(dpt_plan *p, const void *field, const double *poses, const void *cot
     // from the last forward's
     const bool cells = p->cells && pose;
     if (cells) {
-        const int rc = refresh_cells(p, field, s);
+        const int rc = refresh_copy(p, field, s);
         if (rc != DPT_OK) return rc;
     }
     timer_begin(p, 1, s);
@@ -2866,7 +2909,7 @@ int per_ray_vjp(dpt_plan *p, const void *field, const double *poses, const void 
     }
     HIP_TRY(hipGetLastError());
     if (p->cells) {
-        const int rc = refresh_cells(p, field, s);
+        const int rc = refresh_copy(p, field, s);
         if (rc != DPT_OK) return rc;
     }
     p->ray_out = out_rays;

@@ -174,10 +174,11 @@ def _check_extent(decoded: Decoded) -> None:
                     raise ContractError("detector extent exceeds the FP64 finite-ray range")
 
 
-# Largest cell-layout copy (bytes) a plan keeps by default; larger fields
-# gather from the linear array.
+# Largest gather copy (bytes, counted as 8 corners per cell; FP32 copies hold 4
+# per grid sample) a plan keeps by default; larger fields gather from the
+# linear array.
 CELL_GATHER_MAX_BYTES = 32 << 30
-# The copy is rebuilt at every call (about 36 bytes of traffic per cell) and
+# The copy is rebuilt at every call (about 20 bytes of traffic per cell) and
 # saves under a picosecond per sample (full scan: 48 ms over 6.2e10 samples),
 # so a plan takes it only when a call samples at least this many times per
 # cell: the 360-view full scan does (~5800), one 512^2 view of a 512 x 512 x
@@ -186,9 +187,9 @@ CELL_GATHER_MIN_SAMPLES_PER_CELL = 64
 
 
 def gather_cells(decoded: Decoded) -> bool:
-    """FP32 sampling gathers corners from a cell-layout copy of the field
-    (one or two 16-byte loads per cell instead of four 8-byte loads) when a
-    call samples at least CELL_GATHER_MIN_SAMPLES_PER_CELL times per cell and
+    """FP32 sampling gathers corners from a copy of the field (quads in FP32,
+    cells in 16 bits: two or one 16-byte loads per cell instead of four
+    8-byte loads) when a call samples at least CELL_GATHER_MIN_SAMPLES_PER_CELL times per cell and
     the copy fits CELL_GATHER_MAX_BYTES; DPT_AMD_GATHER=linear|cells
     overrides."""
     if decoded.spec.precision != "float32":
