@@ -56,6 +56,7 @@ struct Params {
     int slab_chunks;         // 1: index chunks would overflow even the larger brick often (silhouette-heavy plans)
     int chunk_samples;       // unit of the sample segments
     int gauss_chunks;        // lockstep chunks per ray of the cell-Gauss volume adjoint
+    const double *alpha64;   // 2 x samples entries (FP64 sampling): (k + 0.5) / S, then 1 - that
     const float *alpha;      // 3 x samples entries: alpha_k, k + 0.5, 1 - alpha_k (sample_table_entries)
     int volume_f64;          // 1: FP64 volume destination (increments unflushed, FP64 sampling unrounded)
 };
@@ -464,6 +465,30 @@ __device__ __forceinline__ bool interior32(const Params &P, float p0, float p1, 
     return p0 >= 0.0f && p1 >= 0.0f && p2 >= 0.0f && p0 < P.cx && p1 < P.cy && p2 < P.cz;
 }
 
+// The latest entry ka and the earliest exit kb of the active lanes, within
+// [k0, k1], by bisection (cross-lane reductions would read masked lanes).
+__device__ __forceinline__ void uniform_span(int lo, int hi, int k0, int k1, int &ka, int &kb) {
+    int below = k0, above = k1;
+    while (below < above) {
+        const int m = (below + above) >> 1;
+        if (__builtin_amdgcn_ballot_w64(lo > m) != 0)
+            below = m + 1;
+        else
+            above = m;
+    }
+    ka = below;
+    below = k0;
+    above = k1;
+    while (below < above) {
+        const int m = (below + above + 1) >> 1;
+        if (__builtin_amdgcn_ballot_w64(hi < m) != 0)
+            above = m - 1;
+        else
+            below = m;
+    }
+    kb = below;
+}
+
 // Samples [ka, kb) of [k0, k1) that are interior points for every active lane
 // of the wave (uniform; empty when there are none).  Estimated from the rays'
 // crossings of the planes 0 and n - 1 with a margin of two samples, then both
@@ -483,27 +508,7 @@ __device__ __forceinline__ void interior_span(const Params &P, const float *o, c
     const float per = __builtin_amdgcn_rcpf(step);
     const float lo = fminf(fmaxf(ceilf((enter - lower) * per) + 2.0f, (float)k0), (float)k1);
     const float hi = fminf(fmaxf(floorf((leave - lower) * per) - 2.0f, (float)k0), (float)k1);
-    // the latest entry and the earliest exit of the active lanes, by bisection
-    // (cross-lane reductions would read lanes that this branch masks)
-    int below = k0, above = k1;
-    while (below < above) {
-        const int m = (below + above) >> 1;
-        if (__builtin_amdgcn_ballot_w64((int)lo > m) != 0)
-            below = m + 1;
-        else
-            above = m;
-    }
-    ka = below;
-    below = k0;
-    above = k1;
-    while (below < above) {
-        const int m = (below + above + 1) >> 1;
-        if (__builtin_amdgcn_ballot_w64((int)hi < m) != 0)
-            above = m - 1;
-        else
-            below = m;
-    }
-    kb = below;
+    uniform_span((int)lo, (int)hi, k0, k1, ka, kb);
     if (kb > ka) {
         const float a = fmaf(sample_centre(P, ka), step, lower), b = fmaf(sample_centre(P, kb - 1), step, lower);
         const bool ok = interior32(P, fmaf(a, d[0], o[0]), fmaf(a, d[1], o[1]), fmaf(a, d[2], o[2])) &&
@@ -576,6 +581,14 @@ constexpr int kLayoutScalar = 0;  // linear field, eight scalar loads (nx == 1)
 constexpr int kLayoutPair = 1;    // linear field, x-adjacent pairs (nx > 1)
 constexpr int kLayoutCells = 2;   // cell layout (DPT_STORE_CELLS): one cell per gather
 constexpr int kLayoutQuads = 3;   // quad layout (a plan's own FP32 copy): the cell's two z faces, 4 corners each
+
+// Layout of the plan's copy.  FP32: quads, 16 bytes a load, neighbouring
+// lanes' quads adjacent, half the copy of 32-byte cells (full scan, against
+// cells: forward 57.2 -> 53.8 ms, pose VJP 75.9 -> 72.2, the copy 0.15 -> 0.06).
+// 16-bit: cells, whose one 16-byte load halves the load instructions (24
+// views of 256^2 over 256^3 in bfloat16: forward 2.0 ms, with quads 3.4).
+template <typename T>
+constexpr int kGatherCopy = std::is_same<T, float>::value ? kLayoutQuads : kLayoutCells;
 
 struct __attribute__((aligned(16))) Quad {
     uint32_t x, y, z, w;

@@ -791,7 +791,9 @@ __device__ __forceinline__ void lower_cell64(const Params &P, const double *p, i
 }
 
 // kernels/projection.py:236-274 (weighted lerps; differences before interpolation)
-template <bool GRAD>
+typedef const double __attribute__((address_space(4))) *constant_f64;
+
+template <bool GRAD, bool INTERIOR = false>
 __device__ __forceinline__ double sample_cell64(const Cell64 &c, const double *v, double *g) {
     const double v000 = v[0], v100 = v[1], v010 = v[2], v110 = v[3];
     const double v001 = v[4], v101 = v[5], v011 = v[6], v111 = v[7];
@@ -808,11 +810,71 @@ __device__ __forceinline__ double sample_cell64(const Cell64 &c, const double *v
         const double dy1 = ax * (v011 - v001) + fx * (v111 - v101);
         const double dz0 = ax * (v001 - v000) + fx * (v101 - v100);
         const double dz1 = ax * (v011 - v010) + fx * (v111 - v110);
-        g[0] = c.slx * (az * dx0 + fz * dx1);
-        g[1] = c.sly * (az * dy0 + fz * dy1);
-        g[2] = c.slz * (ay * dz0 + fy * dz1);
+        g[0] = az * dx0 + fz * dx1;
+        g[1] = az * dy0 + fz * dy1;
+        g[2] = ay * dz0 + fy * dz1;
+        if constexpr (!INTERIOR) {
+            g[0] = c.slx * g[0];
+            g[1] = c.sly * g[1];
+            g[2] = c.slz * g[2];
+        }
     }
     return value;
+}
+
+// A point in [0, n - 1) on every axis: cell64's cell and fractions without its
+// clamps, caps and support test (fract(p) = p - floor(p) is exact for p >= 0).
+__device__ __forceinline__ void cell64_interior(const Params &P, const double *p, Cell64 &c) {
+    c.lx = (int)p[0];
+    c.ly = (int)p[1];
+    c.lz = (int)p[2];
+    c.fx = __builtin_amdgcn_fract(p[0]);
+    c.fy = __builtin_amdgcn_fract(p[1]);
+    c.fz = __builtin_amdgcn_fract(p[2]);
+    c.slx = c.sly = c.slz = 1.0;
+    c.base = (c.lz * P.ny + c.ly) * P.nx + c.lx;
+}
+
+// Sample k's position and point, in the reference's unfused arithmetic.
+__device__ __forceinline__ double point64(const Ray &r, double lower, double step, int k, double *p) {
+    const double pos = lower + ((double)k + 0.5) * step;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) p[a] = r.o[a] + pos * r.d[a];
+    return pos;
+}
+
+// interior_span (device_common.h) for FP64 sampling of all samples.  With the
+// interior samples free of clamps, support tests and the division of the
+// sample fraction (tabulated), 24 views of 256^2 over 128^3 at S = 512 run
+// the forward in 1.02 ms (1.35 before) and the pose VJP in 2.21 (2.57); FP64
+// instruction issue bounds both.  (Gathering from a quad copy, as FP32 does,
+// changed neither.)
+__device__ __forceinline__ void interior_span64(const Params &P, const Ray &r, double lower, double step, int &ka,
+                                                int &kb) {
+    const double top[3] = {(double)(P.nx - 1), (double)(P.ny - 1), (double)(P.nz - 1)};
+    float enter = (float)lower, leave = 3e38f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float inverse = __builtin_amdgcn_rcpf((float)r.d[a]);
+        const float u = (float)(0.0 - r.o[a]) * inverse, v = (float)(top[a] - r.o[a]) * inverse;
+        enter = fmaxf(enter, fminf(u, v));
+        leave = fminf(leave, fmaxf(u, v));
+    }
+    const float per = __builtin_amdgcn_rcpf((float)step), count = (float)P.samples;
+    const int lo = (int)fminf(fmaxf(ceilf((enter - (float)lower) * per) + 2.0f, 0.0f), count);
+    const int hi = (int)fminf(fmaxf(floorf((leave - (float)lower) * per) - 2.0f, 0.0f), count);
+    uniform_span(lo, hi, 0, P.samples, ka, kb);
+    if (kb > ka) {
+        bool ok = true;
+        for (int k : {ka, kb - 1}) {
+            double p[3];
+            point64(r, lower, step, k, p);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) ok = ok && p[a] >= 0.0 && p[a] < top[a];
+        }
+        if (__builtin_amdgcn_ballot_w64(!ok) != 0) kb = ka;
+    }
+    if (kb <= ka) ka = kb = P.samples;
 }
 
 // The eight corners as FP64, fetched with the x-pair loads of the FP32 path
@@ -851,23 +913,36 @@ __global__ __launch_bounds__(kBlock) void forward64_kernel(Params P, const T *__
     double integral = 0.0;
     if (iv.upper > iv.lower) {
         const double step = (iv.upper - iv.lower) / (double)P.samples;
-        bool bad = false;
+        // sample points are monotone in the sample index: all are finite iff
+        // the first and the last are
+        double ends[6];
+        point64(r, iv.lower, step, 0, ends);
+        point64(r, iv.lower, step, P.samples - 1, ends + 3);
+        if (!finite3d(ends) || !finite3d(ends + 3)) flag(P, view, DPT_STATUS_RANGE);
         double v[8];
         int cur = -1;  // corners cached while consecutive samples share a cell
-        for (int k = 0; k < P.samples; ++k) {
-            const double pos = iv.lower + ((double)k + 0.5) * step;
-            const double p[3] = {r.o[0] + pos * r.d[0], r.o[1] + pos * r.d[1], r.o[2] + pos * r.d[2]};
-            bad |= !finite3d(p);
-            Cell64 c;
-            if (cell64(P, p, c)) {
+        auto walk = [&](auto interior, int k0, int k1) {
+            for (int k = k0; k < k1; ++k) {
+                double p[3];
+                point64(r, iv.lower, step, k, p);
+                Cell64 c;
+                if constexpr (decltype(interior)::value) {
+                    cell64_interior(P, p, c);
+                } else {
+                    if (!cell64(P, p, c)) continue;
+                }
                 if (c.base != cur) {
                     load8d<T>(P, field, c.base, v);
                     cur = c.base;
                 }
                 integral += sample_cell64<false>(c, v, nullptr);
             }
-        }
-        if (bad) flag(P, view, DPT_STATUS_RANGE);
+        };
+        int ka, kb;
+        interior_span64(P, r, iv.lower, step, ka, kb);
+        walk(std::false_type{}, 0, ka);
+        walk(std::true_type{}, ka, kb);
+        walk(std::false_type{}, kb, P.samples);
         integral *= r.len * step;
     }
     out[ray] = integral;
@@ -912,40 +987,48 @@ __global__ __launch_bounds__(kBlock) void vjp64_kernel(Params P, const T *__rest
             }
         }
     }
-    const bool pow2 = (P.samples & (P.samples - 1)) == 0;
-    const double inverse_samples = pow2 ? 1.0 / S : 0.0;
     double mean = 0.0, dor[3] = {0, 0, 0}, ddir[3] = {0, 0, 0};
     double shift_lower = 0.0, shift_upper = 0.0;
-    bool bad = false;
-
-    double v[8];
-    int cur = -1;  // corners cached while consecutive samples share a cell
     if (active) {
-        for (int k = 0; k < P.samples; ++k) {
-            const double alpha = pow2 ? ((double)k + 0.5) * inverse_samples : ((double)k + 0.5) / S;
-            const double pos = iv.lower + ((double)k + 0.5) * step;
-            const double p[3] = {r.o[0] + pos * r.d[0], r.o[1] + pos * r.d[1], r.o[2] + pos * r.d[2]};
-            bad |= !finite3d(p);
-            Cell64 c;
-            if (!cell64(P, p, c)) continue;
-            double g[3];
-            if (c.base != cur) {
-                load8d<T>(P, field, c.base, v);
-                cur = c.base;
-            }
-            const double value = sample_cell64<true>(c, v, g);
-            mean += value;
+        double ends[6];  // as forward64_kernel
+        point64(r, iv.lower, step, 0, ends);
+        point64(r, iv.lower, step, P.samples - 1, ends + 3);
+        if (!finite3d(ends) || !finite3d(ends + 3)) flag(P, view, DPT_STATUS_RANGE);
+        double v[8];
+        int cur = -1;  // corners cached while consecutive samples share a cell
+        auto walk = [&](auto interior, int k0, int k1) {
+            constexpr bool INTERIOR = decltype(interior)::value;
+            for (int k = k0; k < k1; ++k) {
+                double p[3], g[3];
+                const double pos = point64(r, iv.lower, step, k, p);
+                Cell64 c;
+                if constexpr (INTERIOR) {
+                    cell64_interior(P, p, c);
+                } else {
+                    if (!cell64(P, p, c)) continue;
+                }
+                if (c.base != cur) {
+                    load8d<T>(P, field, c.base, v);
+                    cur = c.base;
+                }
+                mean += sample_cell64<true, INTERIOR>(c, v, g);
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                dor[a] += g[a];
-                ddir[a] += pos * g[a];
+                for (int a = 0; a < 3; ++a) {
+                    dor[a] += g[a];
+                    ddir[a] += pos * g[a];
+                }
+                const double along = g[0] * r.d[0] + g[1] * r.d[1] + g[2] * r.d[2];
+                // uniform: scalar loads
+                shift_lower += ((constant_f64)P.alpha64)[P.samples + k] * along;
+                shift_upper += ((constant_f64)P.alpha64)[k] * along;
             }
-            const double along = g[0] * r.d[0] + g[1] * r.d[1] + g[2] * r.d[2];
-            shift_lower += (1.0 - alpha) * along;
-            shift_upper += alpha * along;
-        }
+        };
+        int ka, kb;
+        interior_span64(P, r, iv.lower, step, ka, kb);
+        walk(std::false_type{}, 0, ka);
+        walk(std::true_type{}, ka, kb);
+        walk(std::false_type{}, kb, P.samples);
     }
-    if (bad) flag(P, view, DPT_STATUS_RANGE);
     if (active) {
         const double lower_seed = -mean + span * shift_lower;
         const double upper_seed = mean + span * shift_upper;
@@ -2081,6 +2164,7 @@ struct dpt_plan {
     int partial_segments = 1;              // d_partials holds this many segments' wave partials
     double *d_acc = nullptr;
     float *d_alpha = nullptr;
+    double *d_alpha64 = nullptr;
     unsigned long long *d_count = nullptr;
     bool cell_gauss = false;  // FP64 exact cell-Gauss integration instead of midpoints
     bool cells = false;       // FP32 sampling gathers from the plan's copy: quads (FP32) or cells (16-bit)
@@ -2315,14 +2399,6 @@ Params copy_params(const dpt_plan *p, Params P) {
     return P;
 }
 
-// Layout of the plan's copy.  FP32: quads, 16 bytes a load, neighbouring
-// lanes' quads adjacent, half the copy of 32-byte cells (full scan, against
-// cells: forward 57.2 -> 53.8 ms, pose VJP 75.9 -> 72.2, the copy 0.15 -> 0.06).
-// 16-bit: cells, whose one 16-byte load halves the load instructions (24
-// views of 256^2 over 256^3 in bfloat16: forward 2.0 ms, with quads 3.4).
-template <typename T>
-constexpr int kGatherCopy = std::is_same<T, float>::value ? kLayoutQuads : kLayoutCells;
-
 template <typename T>
 int launch_forward(dpt_plan *p, const Params &P, const void *field, void *out, bool cells, hipStream_t s) {
     const T *f = static_cast<const T *>(field);
@@ -2396,10 +2472,12 @@ int launch_vjp_c(dpt_plan *p, const Params &P, const void *field, const void *se
             launch_vjp32<T, C, kLayoutPair>(p, P, f, sd, pipe, s);
         else
             launch_vjp32<T, C, kLayoutScalar>(p, P, f, sd, pipe, s);
-    } else if (p->cell_gauss) {
+    } else {
         const double *sd = static_cast<const double *>(seeds);
         const size_t lds = (size_t)P.brick_cap * sizeof(double);
-        if (vol && pose)
+        if (!p->cell_gauss)
+            hipLaunchKernelGGL((vjp64_kernel<T, C>), grid, block, 0, s, P, f, sd, partials);
+        else if (vol && pose)
             hipLaunchKernelGGL((vjp_gauss_kernel<T, true, true, C>), grid, block, lds, s, P, f, sd, p->d_acc,
                                partials);
         else if (vol)
@@ -2408,9 +2486,6 @@ int launch_vjp_c(dpt_plan *p, const Params &P, const void *field, const void *se
         else
             hipLaunchKernelGGL((vjp_gauss_kernel<T, false, true, C>), grid, block, 0, s, P, f, sd, p->d_acc,
                                partials);
-    } else {
-        hipLaunchKernelGGL((vjp64_kernel<T, C>), grid, block, 0, s, P, f, static_cast<const double *>(seeds),
-                           partials);
     }
     HIP_TRY(hipGetLastError());
     return DPT_OK;
@@ -2497,6 +2572,7 @@ int dpt_plan_destroy(dpt_plan *p) {
     (void)hipFree(p->d_partials);
     (void)hipFree(p->d_acc);
     (void)hipFree(p->d_alpha);
+    (void)hipFree(p->d_alpha64);
     (void)hipFree(p->d_copy);
     (void)hipFree(p->d_count);
     (void)hipFree(p->d_gather_rays);
@@ -2701,6 +2777,17 @@ int plan_create(const dpt_grid_desc *grid, int32_t views, int32_t rows, int32_t 
             return cleanup(DPT_E_DEVICE, "copy of the sample fractions failed");
     }
     P.alpha = p->d_alpha;
+    if (arithmetic == DPT_ARITH_FP64) {
+        std::vector<double> alpha(2 * (size_t)samples);
+        for (int k = 0; k < samples; ++k) {
+            alpha[k] = ((double)k + 0.5) / (double)samples;
+            alpha[(size_t)samples + k] = 1.0 - alpha[k];
+        }
+        ALLOC(p->d_alpha64, sizeof(double) * alpha.size());
+        if (hipMemcpy(p->d_alpha64, alpha.data(), sizeof(double) * alpha.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return cleanup(DPT_E_DEVICE, "copy of the sample fractions failed");
+    }
+    P.alpha64 = p->d_alpha64;
     for (auto &e : p->ev)
         if (hipEventCreate(&e) != hipSuccess) return cleanup(DPT_E_DEVICE, "event creation failed");
 #undef ALLOC
