@@ -426,13 +426,6 @@ __device__ __forceinline__ void cell32_inside(const Params &P, float p0, float p
                    (unsigned)c.lx);
 }
 
-// Returns false outside the support.
-__device__ __forceinline__ bool cell32(const Params &P, float p0, float p1, float p2, Cell32 &c) {
-    if (!inside32(P, p0, p1, p2)) return false;
-    cell32_inside(P, p0, p1, p2, c);
-    return true;
-}
-
 // Minimum over the wave; every lane must be active.
 __device__ __forceinline__ int wave_min(int v) {
     // rows of 16, then across rows: lane 63 holds the minimum of the wave
@@ -745,23 +738,6 @@ struct Acc<true> {
         return t.s;
     }
 };
-
-// Position of sample k and its interpolation cell; c.base = -1 outside the
-// support (kernels/projection_fp32.py:116-127, 130-140).  CHECK = false skips
-// the support test for a span of samples that span_inside has cleared.
-template <bool CHECK = true>
-__device__ __forceinline__ void sample_at(const Params &P, const float *o, const float *d, float lower, float step,
-                                          int k, float &pos, Cell32 &c) {
-    pos = fmaf(sample_centre(P, k), step, lower);
-    const float p0 = fmaf(pos, d[0], o[0]);
-    const float p1 = fmaf(pos, d[1], o[1]);
-    const float p2 = fmaf(pos, d[2], o[2]);
-    if constexpr (CHECK) {
-        if (!cell32(P, p0, p1, p2, c)) c.base = -1;
-    } else {
-        cell32_inside(P, p0, p1, p2, c);
-    }
-}
 
 // Every sample point of [k0, k1) lies in the support iff the first and the
 // last do: pos_k = RN(c_k * step + lower) is non-decreasing in k (step > 0)

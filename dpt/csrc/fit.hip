@@ -57,8 +57,8 @@ struct FitTable {
 // Ray march of one request ray: L and the 6-component unit-seed Jacobian row.
 // FP32 storage sums plainly (the projector's FP32 VJP arithmetic); 16-bit
 // storage uses blocked compensated sums.
-template <typename T, bool COMPENSATED>
-__device__ __forceinline__ void fit_ray(const Params &P, const T *field, bool cells, const double *pose, int view, int row,
+template <typename T, bool COMPENSATED, int LAYOUT>
+__device__ __forceinline__ void fit_ray(const Params &P, const T *field, const double *pose, int view, int row,
                                         int col, float &L, double *j, bool &valid) {
     World w;
     ray_world(P, pose, view, row, col, w);
@@ -91,52 +91,57 @@ __device__ __forceinline__ void fit_ray(const Params &P, const T *field, bool ce
     // per-sample support tests only for waves with a ray whose end samples
     // leave the support (uniform flag)
     const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, 0, P.samples)) != 0;
-    for (int k = 0; k < P.samples; ++k) {
-        if constexpr (COMPENSATED) {
-            if (k > 0 && (k % kFoldBlock) == 0) {
-                mean.fold();
-                dor0.fold();
-                dor1.fold();
-                dor2.fold();
-                shl.fold();
-                shu.fold();
-                dd0.fold();
-                dd1.fold();
-                dd2.fold();
+    auto walk = [&](auto interior, int k0, int k1) {
+        constexpr bool INTERIOR = decltype(interior)::value;
+        for (int k = k0; k < k1; ++k) {
+            if constexpr (COMPENSATED) {
+                if (k > 0 && (k % kFoldBlock) == 0) {
+                    mean.fold();
+                    dor0.fold();
+                    dor1.fold();
+                    dor2.fold();
+                    shl.fold();
+                    shu.fold();
+                    dd0.fold();
+                    dd1.fold();
+                    dd2.fold();
+                }
             }
+            const float pos = fmaf(sample_centre(P, k), step, iv.lower);
+            const float p0 = fmaf(pos, d[0], o[0]);
+            const float p1 = fmaf(pos, d[1], o[1]);
+            const float p2 = fmaf(pos, d[2], o[2]);
+            Cell32 c;
+            if constexpr (INTERIOR) {
+                cell32_interior(P, p0, p1, p2, c);
+            } else {
+                if (checked && !inside32(P, p0, p1, p2)) continue;
+                cell32_inside(P, p0, p1, p2, c);
+            }
+            if (c.base != cur) {
+                load8<T, LAYOUT>(P, field, c.base, v);
+                cur = c.base;
+            }
+            float wt[8], g[3];
+            weights32(c, wt);
+            mean.add(interpolate32(wt, v));
+            slopes32(c, v, g);
+            dor0.add(g[0]);
+            dor1.add(g[1]);
+            dor2.add(g[2]);
+            dd0.fma_add(pos, g[0]);
+            dd1.fma_add(pos, g[1]);
+            dd2.fma_add(pos, g[2]);
+            const float along = fmaf(g[2], d[2], fmaf(g[1], d[1], g[0] * d[0]));
+            shl.fma_add(sample_beta(P, k), along);
+            shu.fma_add(sample_alpha(P, k), along);
         }
-        float pos;
-        Cell32 c;
-        if (checked) {
-            sample_at<true>(P, o, d, iv.lower, step, k, pos, c);
-            if (c.base < 0) continue;
-        } else {
-            sample_at<false>(P, o, d, iv.lower, step, k, pos, c);
-        }
-        if (c.base != cur) {
-            if (cells)
-                load8<T, kLayoutCells>(P, field, c.base, v);
-            else if (P.sx)
-                load8<T, kLayoutPair>(P, field, c.base, v);
-            else
-                load8<T, kLayoutScalar>(P, field, c.base, v);
-            cur = c.base;
-        }
-        float wt[8], g[3];
-        weights32(c, wt);
-        mean.add(interpolate32(wt, v));
-        slopes32(c, v, g);
-        dor0.add(g[0]);
-        dor1.add(g[1]);
-        dor2.add(g[2]);
-        dd0.fma_add(pos, g[0]);
-        dd1.fma_add(pos, g[1]);
-        dd2.fma_add(pos, g[2]);
-        const float alpha = sample_alpha(P, k);
-        const float along = fmaf(g[2], d[2], fmaf(g[1], d[1], g[0] * d[0]));
-        shl.fma_add(1.0f - alpha, along);
-        shu.fma_add(alpha, along);
-    }
+    };
+    int ka, kb;
+    interior_span(P, o, d, iv.lower, step, 0, P.samples, ka, kb);
+    walk(std::false_type{}, 0, ka);
+    walk(std::true_type{}, ka, kb);
+    walk(std::false_type{}, kb, P.samples);
     const float m = mean.value();
     L = m * (len * step);
     const float lower_seed = fmaf(span, shl.value(), -m);
@@ -156,17 +161,35 @@ __device__ __forceinline__ void fit_ray(const Params &P, const T *field, bool ce
     pose_epilogue<6>(P, pose, w, (double)len / (double)P.samples, og, dg, j);
 }
 
+template <typename T, bool COMPENSATED>
+__device__ __forceinline__ void fit_ray_in(const Params &P, const void *field, bool cells, const double *pose, int view,
+                                           int row, int col, float &L, double *j, bool &valid) {
+    const T *f = static_cast<const T *>(field);
+    if (cells)
+        fit_ray<T, COMPENSATED, kLayoutCells>(P, f, pose, view, row, col, L, j, valid);
+    else if (P.sx)
+        fit_ray<T, COMPENSATED, kLayoutPair>(P, f, pose, view, row, col, L, j, valid);
+    else
+        fit_ray<T, COMPENSATED, kLayoutScalar>(P, f, pose, view, row, col, L, j, valid);
+}
+
+// Persistent waves: each pulls one 8x8 quarter of a 16x16 tile at a time from
+// the counter, so the waves of a tile whose rays miss the volume move on and
+// the last round is short; the unit is uniform over the wave, so its request
+// is read with scalar loads.  VALU issue bounds the march.  Six requests of 3
+// views of 192^2 on 128^3 bfloat16 cells at S = 384: 0.72 ms a step when
+// workgroups pulled whole tiles, 0.53 ms now (interior samples included).
 __global__ __launch_bounds__(kBlock) void fit_step_kernel(const FitTable *__restrict__ tab,
                                                           double *__restrict__ partials, int *counter) {
-    __shared__ int next;
-    const int total = tab->total_tiles;
+    const int total = 4 * tab->total_tiles;
     const int n = tab->n_requests;
+    const int l = threadIdx.x & 63;
     while (true) {
-        if (threadIdx.x == 0) next = atomicAdd(counter, 1);
-        __syncthreads();
-        const int t = next;
-        __syncthreads();
-        if (t >= total) break;
+        int unit = 0;
+        if (l == 0) unit = atomicAdd(counter, 1);
+        unit = __builtin_amdgcn_readfirstlane(unit);
+        if (unit >= total) break;
+        const int t = unit >> 2, w = unit & 3;
         // request owning tile t: largest r with tile_begin[r] <= t
         int lo = 0, hi = n - 1;
         while (lo < hi) {
@@ -182,7 +205,6 @@ __global__ __launch_bounds__(kBlock) void fit_step_kernel(const FitTable *__rest
         const int view = local / P.tiles_per_group;
         const int rem = local - view * P.tiles_per_group;
         const int ty = rem / P.tiles_x, tx = rem - (rem / P.tiles_x) * P.tiles_x;
-        const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
         const int row = ty * kTile + (w >> 1) * 8 + (l >> 3);
         const int col = tx * kTile + (w & 1) * 8 + (l & 7);
         double acc[kFitTerms];
@@ -195,14 +217,11 @@ __global__ __launch_bounds__(kBlock) void fit_step_kernel(const FitTable *__rest
             const int element = R.storage & ~DPT_STORE_CELLS;
             const bool cells = (R.storage & DPT_STORE_CELLS) != 0;
             if (element == DPT_STORE_BF16)
-                fit_ray<__hip_bfloat16, true>(P, static_cast<const __hip_bfloat16 *>(R.field), cells, R.state, view,
-                                              row, col, L, jr, valid);
+                fit_ray_in<__hip_bfloat16, true>(P, R.field, cells, R.state, view, row, col, L, jr, valid);
             else if (element == DPT_STORE_F16)
-                fit_ray<__half, true>(P, static_cast<const __half *>(R.field), cells, R.state, view, row, col, L, jr,
-                                      valid);
+                fit_ray_in<__half, true>(P, R.field, cells, R.state, view, row, col, L, jr, valid);
             else
-                fit_ray<float, false>(P, static_cast<const float *>(R.field), cells, R.state, view, row, col, L, jr,
-                                      valid);
+                fit_ray_in<float, false>(P, R.field, cells, R.state, view, row, col, L, jr, valid);
             const double res = (double)L - (double)R.targets[((size_t)view * P.rows + row) * P.cols + col];
             int q = 0;
 #pragma unroll
@@ -213,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void fit_step_kernel(const FitTable *__rest
             for (int a = 0; a < 6; ++a) acc[21 + a] = jr[a] * res;
             acc[27] = res * res;
         }
-        double *out = partials + ((size_t)t * 4 + w) * kFitTerms;
+        double *out = partials + (size_t)unit * kFitTerms;
 #pragma unroll
         for (int i = 0; i < kFitTerms; ++i) {
             const double s = wave_sum(acc[i]);
@@ -283,26 +302,33 @@ __global__ __launch_bounds__(kBlock) void fit_update_kernel(const FitTable *__re
     if (r == 0 && threadIdx.x == 0) *counter = 0;  // re-arm the tile counter for the next step
     if (r >= tab->n_requests) return;
     const size_t begin = (size_t)tab->tile_begin[r] * 4, end = (size_t)tab->tile_begin[r + 1] * 4;
-    __shared__ double red[kBlock];
-    __shared__ double sums[kFitTerms];
-    for (int i = 0; i < kFitTerms; ++i) {
-        double v = 0.0;
-        for (size_t p = begin + threadIdx.x; p < end; p += kBlock) v += partials[p * kFitTerms + i];
-        red[threadIdx.x] = v;
-        __syncthreads();
-        for (int s = kBlock / 2; s > 0; s >>= 1) {
-            if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-            __syncthreads();
+    // every term at once: per-thread strided sums, then one pairwise tree per
+    // term (the order of a term-by-term pass, which took 57 us in place of
+    // 16)
+    __shared__ double red[kFitTerms][kBlock];
+    double v[kFitTerms];
+#pragma unroll
+    for (int i = 0; i < kFitTerms; ++i) v[i] = 0.0;
+    for (size_t p = begin + threadIdx.x; p < end; p += kBlock) {
+#pragma unroll
+        for (int i = 0; i < kFitTerms; ++i) v[i] += partials[p * kFitTerms + i];
+    }
+#pragma unroll
+    for (int i = 0; i < kFitTerms; ++i) red[i][threadIdx.x] = v[i];
+    __syncthreads();
+    for (int s = kBlock / 2; s > 0; s >>= 1) {
+        if (threadIdx.x < s) {
+#pragma unroll
+            for (int i = 0; i < kFitTerms; ++i) red[i][threadIdx.x] += red[i][threadIdx.x + s];
         }
-        if (threadIdx.x == 0) sums[i] = red[0];
         __syncthreads();
     }
     if (threadIdx.x != 0) return;
     double *st = tab->req[r].state;
-    const double loss = 0.5 * sums[27];
+    const double loss = 0.5 * red[27][0];
     double A[21], b[6];
-    for (int i = 0; i < 21; ++i) A[i] = sums[i];
-    for (int i = 0; i < 6; ++i) b[i] = sums[21 + i];
+    for (int i = 0; i < 21; ++i) A[i] = red[i][0];
+    for (int i = 0; i < 6; ++i) b[i] = red[21 + i][0];
     const double evals = st[DPT_FIT_EVALS];
     double lambda = st[DPT_FIT_LAMBDA];
     if (evals == 0.0 || (isfinite(loss) && loss <= st[DPT_FIT_BEST_LOSS])) {
