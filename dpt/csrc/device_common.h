@@ -42,7 +42,8 @@ struct Params {
     int vb;                  // views per workgroup (1, 2 or 4): one wave64 per view when > 1
     int tile_w, tile_h;      // pixels per workgroup tile of one view
     int tiles_x, tiles_y, tiles_per_group, total_tiles, chunk;
-    int segments;            // FP32 VJP: workgroups per tile, each over its own range of samples
+    int by_rows;             // 1: XCDs take rows of tiles in turn, not contiguous runs of the walk
+    int segments;            // volume adjoint: workgroups per tile, each over its own range of samples
     int base_tiles;          // tiles of one segment (total_tiles / segments)
     int segment_samples;     // samples per segment (a multiple of chunk_samples)
     int wt_x, wt_y, wt_per_view;  // wave tiles (8x8 pixels, or 64 rays) per view
@@ -117,10 +118,23 @@ __device__ __forceinline__ bool finite3d(const double *v) {
 // per view).  Each wave owns one 8x8 wave tile of one view; `wslot` indexes its
 // pose partials.  Explicit ray bundles use 256 consecutive rays per workgroup.
 // Returns false when the whole workgroup lies past the end of the walk.
+//
+// Launches of few views hand out single rows of tiles instead (P.by_rows):
+// rays that meet the volume crowd the middle of a panel, so contiguous runs
+// left most XCDs idle.  One 512^2 view of a
+// 512 x 512 x 139 grid, whole call: 2.76 -> 1.98 ms; 24 views and more keep the
+// runs, whose L2s hold a part of the volume each (FP64 24 x 256^2 over 128^3:
+// 4.7 ms, by rows 5.8).
+__device__ __forceinline__ int walk_index(int b, int chunk, int row, bool by_rows) {
+    const int xcd = b % kXcds, i = b / kXcds;
+    return by_rows ? ((i / row) * kXcds + xcd) * row + i % row : xcd * chunk + i;
+}
+__device__ __forceinline__ int tile_index(const Params &P) {
+    return walk_index(blockIdx.x, P.chunk, P.tiles_x, P.by_rows);
+}
 __device__ __forceinline__ bool lane_ray(const Params &P, int &view, int &row, int &col, int &wslot,
                                          bool &wave_valid) {
-    const int b = blockIdx.x;
-    int logical = (b % kXcds) * P.chunk + b / kXcds;
+    int logical = tile_index(P);
     if (logical >= P.total_tiles) return false;
     if (P.segments > 1) logical %= P.base_tiles;  // segment logical / base_tiles
     const int group = logical / P.tiles_per_group;

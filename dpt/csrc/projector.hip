@@ -50,22 +50,10 @@
 
 namespace dpt {
 
-// PIPE (FP32 storage; forward and pose-only VJP): the samples of a ray in one
-// software pipeline, the corner loads of sample k + kPipeDepth issued before sample k
-// is summed.  Small launches (one wave per SIMD or fewer) expose a memory
-// latency per sample; this hides it without splitting the ray, so each pose
-// sum stays the reference's one sequential FP32 sum (forward: the same
-// sequential sum of interpolated values).  Eight slots of corner
-// values, fractions and positions take 220 VGPRs (two waves per SIMD); on a
-// one-view 512^2 launch depth 8 ran the pose VJP in 0.61 ms (central-window
-// cotangent) and 0.84 ms (every ray), depth 4 in 0.86 / 1.31 ms, and
-// recomputing the cell at the sum instead of keeping it was slower.
-constexpr int kPipeDepth = 8;
-
 // ------------------------------------------------------- FP32 forward ------
 // kernels/projection_fp32.py:334-374
 
-template <typename T, bool COMPENSATED, int LAYOUT, bool PIPE = false>
+template <typename T, bool COMPENSATED, int LAYOUT>
 __global__ __launch_bounds__(kBlock) void forward32_kernel(Params P, const T *__restrict__ field,
                                                            float *__restrict__ out) {
     int view, row, col, wslot;
@@ -125,69 +113,15 @@ __global__ __launch_bounds__(kBlock) void forward32_kernel(Params P, const T *__
                 total.add(interpolate32(wt, v));
             }
         };
-        static_assert(!PIPE || !COMPENSATED, "the pipeline is an FP32-storage loop");
-        if constexpr (PIPE) {
-            // slot j: corner values, fractions and support flag of the sample
-            // issued kPipeDepth samples back; an outside sample adds -0, the
-            // identity of FP32 addition (the reference skips it)
-            float ring[kPipeDepth][8], rf[kPipeDepth][3], cur[8];
-            bool rin[kPipeDepth], fresh[kPipeDepth];
-            int prev = -1;
-            auto issue = [&](int j, int k) {
-                const float pos = fmaf(sample_centre(P, k), step, iv.lower);
-                const float p0 = fmaf(pos, d[0], o[0]);
-                const float p1 = fmaf(pos, d[1], o[1]);
-                const float p2 = fmaf(pos, d[2], o[2]);
-                Cell32 c;
-                cell32_inside(P, p0, p1, p2, c);  // clamped: the load stays in the field
-                rin[j] = inside32(P, p0, p1, p2);
-                rf[j][0] = c.fx;
-                rf[j][1] = c.fy;
-                rf[j][2] = c.fz;
-                // only lanes whose cell changed since the previous sample load
-                fresh[j] = c.base != prev;
-                prev = c.base;
-                if (fresh[j]) load8<T, LAYOUT>(P, field, c.base, ring[j]);
-            };
-            auto consume = [&](int j) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) cur[q] = fresh[j] ? ring[j][q] : cur[q];
-                Cell32 c;
-                c.fx = rf[j][0];
-                c.fy = rf[j][1];
-                c.fz = rf[j][2];
-                float wt[8];
-                weights32(c, wt);
-                const float value = interpolate32(wt, cur);
-                total.add(rin[j] ? value : -0.0f);
-            };
-#pragma unroll
-            for (int q = 0; q < 8; ++q) cur[q] = 0.0f;
-            const int last = P.samples;
-#pragma unroll
-            for (int j = 0; j < kPipeDepth; ++j) issue(j, min(j, last - 1));
-            int k0 = 0;
-            for (; k0 + kPipeDepth <= last; k0 += kPipeDepth) {
-#pragma unroll
-                for (int j = 0; j < kPipeDepth; ++j) {
-                    consume(j);
-                    issue(j, min(k0 + j + kPipeDepth, last - 1));
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < kPipeDepth; ++j)
-                if (k0 + j < last) consume(j);  // uniform
-        } else {
-            // per-sample support tests only for waves with a ray whose end
-            // samples leave the support; clamps only outside the samples that
-            // are interior points for the whole wave
-            const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, 0, P.samples)) != 0;
-            int ka, kb;
-            interior_span(P, o, d, iv.lower, step, 0, P.samples, ka, kb);
-            walk(std::false_type{}, 0, ka, checked);
-            walk(std::true_type{}, ka, kb, false);
-            walk(std::false_type{}, kb, P.samples, checked);
-        }
+        // per-sample support tests only for waves with a ray whose end
+        // samples leave the support; clamps only outside the samples that
+        // are interior points for the whole wave
+        const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, 0, P.samples)) != 0;
+        int ka, kb;
+        interior_span(P, o, d, iv.lower, step, 0, P.samples, ka, kb);
+        walk(std::false_type{}, 0, ka, checked);
+        walk(std::true_type{}, ka, kb, false);
+        walk(std::false_type{}, kb, P.samples, checked);
         if (bad) flag(P, view, DPT_STATUS_RANGE);
         result = total.value() * (len * step);
     }
@@ -510,6 +444,83 @@ __device__ __forceinline__ void drain_brick(const Params &P, const Brick &B, dou
     }
 }
 
+// The nine sums of a ray's pose adjoint, in sample order.
+template <bool COMPENSATED>
+struct PoseSums {
+    Acc<COMPENSATED> mean, dor0, dor1, dor2, dd0, dd1, dd2, shl, shu;
+    __device__ __forceinline__ void init() {
+        mean.init();
+        dor0.init();
+        dor1.init();
+        dor2.init();
+        dd0.init();
+        dd1.init();
+        dd2.init();
+        shl.init();
+        shu.init();
+    }
+    __device__ __forceinline__ void fold() {
+        mean.fold();
+        dor0.fold();
+        dor1.fold();
+        dor2.fold();
+        dd0.fold();
+        dd1.fold();
+        dd2.fold();
+        shl.fold();
+        shu.fold();
+    }
+    // sample k at position pos with value and slopes
+    __device__ __forceinline__ void add(const Params &P, int k, float pos, float value, float g0, float g1, float g2,
+                                        const float *d) {
+        mean.add(value);
+        dor0.add(g0);
+        dor1.add(g1);
+        dor2.add(g2);
+        // contracted by the reference's code generator (fuse_fp)
+        dd0.fma_add(pos, g0);
+        dd1.fma_add(pos, g1);
+        dd2.fma_add(pos, g2);
+        const float along = fmaf(g2, d[2], fmaf(g1, d[1], g0 * d[0]));
+        shl.fma_add(sample_beta(P, k), along);
+        shu.fma_add(sample_alpha(P, k), along);
+    }
+};
+
+// A ray's pose gradient from its sums (all zero for an inactive ray), stored
+// or reduced over the wave.
+template <int C, bool COMPENSATED>
+__device__ __forceinline__ void pose_finish(const Params &P, const double *pose, bool active,
+                                            const PoseSums<COMPENSATED> &q, const Interval32 &iv, float len, float seed,
+                                            float span, float step, double *partials, int wslot, bool wave_valid,
+                                            int view, int row, int col) {
+    double gradient[kMaxComponents];
+#pragma unroll
+    for (int c = 0; c < kMaxComponents; ++c) gradient[c] = 0.0;
+    if (active) {
+        const float m = q.mean.value();
+        const float lower_seed = fmaf(span, q.shl.value(), -m);
+        const float upper_seed = fmaf(span, q.shu.value(), m);
+        const float dor[3] = {q.dor0.value(), q.dor1.value(), q.dor2.value()};
+        const float ddir[3] = {q.dd0.value(), q.dd1.value(), q.dd2.value()};
+        double og[3], dg[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float lo_o = (iv.lo_axis == a) ? iv.lo_o : 0.0f;
+            const float lo_d = (iv.lo_axis == a) ? iv.lo_d : 0.0f;
+            const float up_o = (iv.up_axis == a) ? iv.up_o : 0.0f;
+            const float up_d = (iv.up_axis == a) ? iv.up_d : 0.0f;
+            og[a] = (double)fmaf(upper_seed, up_o, fmaf(lower_seed, lo_o, span * dor[a]));
+            dg[a] = (double)fmaf(upper_seed, up_d, fmaf(lower_seed, lo_d, span * ddir[a]));
+        }
+        const float factor = (seed * len) / (float)P.samples;
+        World w;  // recomputed: keeps 24 FP64 registers out of the sample loop
+        ray_world(P, pose, view, row, col, w);
+        pose_epilogue<C>(P, pose, w, (double)factor, og, dg, gradient, (double)seed, (double)(m * step));
+    }
+    store_gradient<C>(P, gradient, partials, wslot, wave_valid, view, row, col);
+}
+
 // ----------------------------------------------------- FP32 pose VJP ------
 // kernels/projection_fp32.py:377-617, the pose half: each lane marches its ray
 // once and sums the interpolated values, the slopes and the clip-face terms in
@@ -517,7 +528,7 @@ __device__ __forceinline__ void drain_brick(const Params &P, const Brick &B, dou
 // support (only waves whose rays' end samples leave it test per sample) take
 // the clamped cell with zero value and slopes: they add nothing, as the
 // reference skips them.
-template <typename T, int C, bool COMPENSATED, int LAYOUT, bool PIPE = false>
+template <typename T, int C, bool COMPENSATED, int LAYOUT>
 __global__ __launch_bounds__(kBlock) void vjp32_kernel(Params P, const T *__restrict__ field,
                                                        const float *__restrict__ seeds,
                                                        double *__restrict__ partials) {
@@ -525,16 +536,6 @@ __global__ __launch_bounds__(kBlock) void vjp32_kernel(Params P, const T *__rest
     bool wave_valid;
     if (!lane_ray(P, view, row, col, wslot, wave_valid)) return;
     const double *pose = P.poses + 12 * (size_t)view;
-    // this workgroup's samples [first, last) and its pose partial slot
-    int first = 0, last = P.samples;
-    if (P.segments > 1) {
-        const int b = blockIdx.x;
-        const int seg = ((b % kXcds) * P.chunk + b / kXcds) / P.base_tiles;
-        first = seg * P.segment_samples;
-        last = min(first + P.segment_samples, P.samples);
-        wslot += (view * (P.segments - 1) + seg) * P.wt_per_view;
-    }
-
     // ---- per-ray setup
     bool active = false, bad = false;
     float o[3] = {0, 0, 0}, d[3] = {0, 0, 0}, len = 0.0f, seed = 0.0f, span = 0.0f, step = 0.0f;
@@ -570,182 +571,325 @@ __global__ __launch_bounds__(kBlock) void vjp32_kernel(Params P, const T *__rest
         }
     }
 
-    Acc<COMPENSATED> mean, dor0, dor1, dor2, dd0, dd1, dd2, shl, shu;
-    mean.init();
-    dor0.init();
-    dor1.init();
-    dor2.init();
-    dd0.init();
-    dd1.init();
-    dd2.init();
-    shl.init();
-    shu.init();
-
-    static_assert(!PIPE || !COMPENSATED, "the pipeline is an FP32-storage loop");
+    PoseSums<COMPENSATED> q;
+    q.init();
     if (active) {
-        if constexpr (PIPE) {
-                // slot j holds sample k's corner values, fractions, slopes,
-                // position and support flag from its issue kPipeDepth samples back
-                float ring[kPipeDepth][8], rf[kPipeDepth][6], rpos[kPipeDepth], rlive[kPipeDepth];
-                auto issue = [&](int j, int k) {
-                    const float pos = fmaf(sample_centre(P, k), step, iv.lower);
-                    const float p0 = fmaf(pos, d[0], o[0]);
-                    const float p1 = fmaf(pos, d[1], o[1]);
-                    const float p2 = fmaf(pos, d[2], o[2]);
-                    Cell32 c;
-                    cell32_inside(P, p0, p1, p2, c);  // clamped: the load stays in the field
-                    const bool inside = inside32(P, p0, p1, p2);
-                    rf[j][0] = inside ? c.fx : 0.0f;
-                    rf[j][1] = inside ? c.fy : 0.0f;
-                    rf[j][2] = inside ? c.fz : 0.0f;
-                    rf[j][3] = inside ? c.slx : 0.0f;
-                    rf[j][4] = inside ? c.sly : 0.0f;
-                    rf[j][5] = inside ? c.slz : 0.0f;
-                    rpos[j] = pos;
-                    rlive[j] = inside ? 1.0f : 0.0f;
-                    load8<T, LAYOUT>(P, field, c.base, ring[j]);
-                };
-                auto consume = [&](int j, int k) {
-                    Cell32 c;
-                    c.fx = rf[j][0];
-                    c.fy = rf[j][1];
-                    c.fz = rf[j][2];
-                    c.slx = rf[j][3];
-                    c.sly = rf[j][4];
-                    c.slz = rf[j][5];
-                    float wt[8], g[3];
-                    weights32(c, wt);
-                    const float value = interpolate32(wt, ring[j]) * rlive[j];
-                    slopes32(c, ring[j], g);
-                    const float pos = rpos[j];
-                    mean.add(value);
-                    dor0.add(g[0]);
-                    dor1.add(g[1]);
-                    dor2.add(g[2]);
-                    dd0.fma_add(pos, g[0]);
-                    dd1.fma_add(pos, g[1]);
-                    dd2.fma_add(pos, g[2]);
-                    const float alpha = sample_alpha(P, k);
-                    const float along = fmaf(g[2], d[2], fmaf(g[1], d[1], g[0] * d[0]));
-                    shl.fma_add(1.0f - alpha, along);
-                    shu.fma_add(alpha, along);
-                };
-    #pragma unroll
-                for (int j = 0; j < kPipeDepth; ++j) issue(j, min(first + j, last - 1));
-                // whole groups without branches, so that the loads stay in flight
-                // across iterations; the last group's issues repeat sample
-                // last - 1 and are not consumed
-                int k0 = first;
-                for (; k0 + kPipeDepth <= last; k0 += kPipeDepth) {
-    #pragma unroll
-                    for (int j = 0; j < kPipeDepth; ++j) {
-                        consume(j, k0 + j);
-                        issue(j, min(k0 + j + kPipeDepth, last - 1));
+        float v[8];
+        int cur = -1;
+        auto walk = [&](auto interior, int k0, int k1, bool checked) {
+            constexpr bool INTERIOR = decltype(interior)::value;
+            for (int k = k0; k < k1; ++k) {
+                if constexpr (COMPENSATED) {
+                    if (k > 0 && (k % kFoldBlock) == 0) q.fold();
+                }
+                const float pos = fmaf(sample_centre(P, k), step, iv.lower);
+                const float p0 = fmaf(pos, d[0], o[0]);
+                const float p1 = fmaf(pos, d[1], o[1]);
+                const float p2 = fmaf(pos, d[2], o[2]);
+                Cell32 c;
+                float live = 1.0f;
+                if constexpr (INTERIOR) {
+                    cell32_interior(P, p0, p1, p2, c);
+                } else {
+                    cell32_inside(P, p0, p1, p2, c);
+                    if (checked) {  // outside samples add nothing
+                        const bool inside = inside32(P, p0, p1, p2);
+                        c.fx = inside ? c.fx : 0.0f;
+                        c.fy = inside ? c.fy : 0.0f;
+                        c.fz = inside ? c.fz : 0.0f;
+                        c.slx = inside ? c.slx : 0.0f;
+                        c.sly = inside ? c.sly : 0.0f;
+                        c.slz = inside ? c.slz : 0.0f;
+                        live = inside ? 1.0f : 0.0f;
                     }
                 }
-    #pragma unroll
-                for (int j = 0; j < kPipeDepth; ++j)
-                    if (k0 + j < last) consume(j, k0 + j);  // uniform
-        } else {
-            float v[8];
-            int cur = -1;
-            auto walk = [&](auto interior, int k0, int k1, bool checked) {
-                constexpr bool INTERIOR = decltype(interior)::value;
-                for (int k = k0; k < k1; ++k) {
-                    if constexpr (COMPENSATED) {
-                        if (k > first && ((k - first) % kFoldBlock) == 0) {
-                            mean.fold();
-                            dor0.fold();
-                            dor1.fold();
-                            dor2.fold();
-                            dd0.fold();
-                            dd1.fold();
-                            dd2.fold();
-                            shl.fold();
-                            shu.fold();
-                        }
-                    }
-                    const float pos = fmaf(sample_centre(P, k), step, iv.lower);
-                    const float p0 = fmaf(pos, d[0], o[0]);
-                    const float p1 = fmaf(pos, d[1], o[1]);
-                    const float p2 = fmaf(pos, d[2], o[2]);
-                    Cell32 c;
-                    float live = 1.0f;
-                    if constexpr (INTERIOR) {
-                        cell32_interior(P, p0, p1, p2, c);
-                    } else {
-                        cell32_inside(P, p0, p1, p2, c);
-                        if (checked) {  // outside samples add nothing
-                            const bool inside = inside32(P, p0, p1, p2);
-                            c.fx = inside ? c.fx : 0.0f;
-                            c.fy = inside ? c.fy : 0.0f;
-                            c.fz = inside ? c.fz : 0.0f;
-                            c.slx = inside ? c.slx : 0.0f;
-                            c.sly = inside ? c.sly : 0.0f;
-                            c.slz = inside ? c.slz : 0.0f;
-                            live = inside ? 1.0f : 0.0f;
-                        }
-                    }
-                    if (c.base != cur) {
-                        load8<T, LAYOUT>(P, field, c.base, v);
-                        cur = c.base;
-                    }
-                    float wt[8], g[3];
-                    weights32(c, wt);
-                    // an outside sample's slopes are zero (above); its value is zeroed here
-                    const float value = INTERIOR ? interpolate32(wt, v) : interpolate32(wt, v) * live;
-                    slopes32(c, v, g);
-                    mean.add(value);
-                    dor0.add(g[0]);
-                    dor1.add(g[1]);
-                    dor2.add(g[2]);
-                    // contracted by the reference's code generator (fuse_fp)
-                    dd0.fma_add(pos, g[0]);
-                    dd1.fma_add(pos, g[1]);
-                    dd2.fma_add(pos, g[2]);
-                    const float along = fmaf(g[2], d[2], fmaf(g[1], d[1], g[0] * d[0]));
-                    shl.fma_add(sample_beta(P, k), along);
-                    shu.fma_add(sample_alpha(P, k), along);
+                if (c.base != cur) {
+                    load8<T, LAYOUT>(P, field, c.base, v);
+                    cur = c.base;
                 }
-            };
-            // per-sample support tests only for waves with a ray whose end
-            // samples leave the support (uniform over the wave); clamps and
-            // slope flags only outside the samples that are interior points
-            // for the whole wave (full scan: 86.9 -> 75.9 ms)
-            const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, first, last)) != 0;
-            int ka, kb;
-            interior_span(P, o, d, iv.lower, step, first, last, ka, kb);
-            walk(std::false_type{}, first, ka, checked);
-            walk(std::true_type{}, ka, kb, false);
-            walk(std::false_type{}, kb, last, checked);
-        }
+                float wt[8], g[3];
+                weights32(c, wt);
+                // an outside sample's slopes are zero (above); its value is zeroed here
+                const float value = INTERIOR ? interpolate32(wt, v) : interpolate32(wt, v) * live;
+                slopes32(c, v, g);
+                q.add(P, k, pos, value, g[0], g[1], g[2], d);
+            }
+        };
+        // per-sample support tests only for waves with a ray whose end
+        // samples leave the support (uniform over the wave); clamps and
+        // slope flags only outside the samples that are interior points
+        // for the whole wave (full scan: 86.9 -> 75.9 ms)
+        const bool checked = __builtin_amdgcn_ballot_w64(!span_inside(P, o, d, iv.lower, step, 0, P.samples)) != 0;
+        int ka, kb;
+        interior_span(P, o, d, iv.lower, step, 0, P.samples, ka, kb);
+        walk(std::false_type{}, 0, ka, checked);
+        walk(std::true_type{}, ka, kb, false);
+        walk(std::false_type{}, kb, P.samples, checked);
     }
-    double gradient[kMaxComponents];
-#pragma unroll
-    for (int c = 0; c < kMaxComponents; ++c) gradient[c] = 0.0;
-    if (active) {
-        const float m = mean.value();
-        const float lower_seed = fmaf(span, shl.value(), -m);
-        const float upper_seed = fmaf(span, shu.value(), m);
-        const float dor[3] = {dor0.value(), dor1.value(), dor2.value()};
-        const float ddir[3] = {dd0.value(), dd1.value(), dd2.value()};
-        double og[3], dg[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float lo_o = (iv.lo_axis == a) ? iv.lo_o : 0.0f;
-            const float lo_d = (iv.lo_axis == a) ? iv.lo_d : 0.0f;
-            const float up_o = (iv.up_axis == a) ? iv.up_o : 0.0f;
-            const float up_d = (iv.up_axis == a) ? iv.up_d : 0.0f;
-            og[a] = (double)fmaf(upper_seed, up_o, fmaf(lower_seed, lo_o, span * dor[a]));
-            dg[a] = (double)fmaf(upper_seed, up_d, fmaf(lower_seed, lo_d, span * ddir[a]));
-        }
-        const float factor = (seed * len) / (float)P.samples;
-        World w;  // recomputed: keeps 24 FP64 registers out of the sample loop
-        ray_world(P, pose, view, row, col, w);
-        pose_epilogue<C>(P, pose, w, (double)factor, og, dg, gradient, (double)seed, (double)(m * step));
-    }
-    store_gradient<C>(P, gradient, partials, wslot, wave_valid, view, row, col);
+    pose_finish<C, COMPENSATED>(P, pose, active, q, iv, len, seed, span, step, partials, wslot, wave_valid, view, row,
+                                col);
     if (bad) flag(P, view, DPT_STATUS_RANGE);
+}
+
+// ------------------------------------------------ FP32 small launches -----
+// A launch of few rays (one 512^2 view is four waves per SIMD) leaves the
+// march of a lane per ray exposed to the memory latency of every sample.
+// Here a workgroup of eight waves holds 64 rays: seven waves sample, each
+// kSplitRun consecutive samples a round with their loads in flight together,
+// and leave values (and slopes) in LDS; the eighth adds the previous round's in
+// sample order, so every sum is the sequential sum of the one-lane march, bit
+// for bit.  Adding costs about 14 of the 85 instructions of a pose sample,
+// hence the ratio.  MI355X, against a software pipeline of 8 samples in one
+// lane: one 512^2 view of a 512 x 512 x 139 grid at S = 1024 (with rows of
+// tiles dealt to the XCDs) forward 555 -> 268 us, pose VJP 1350 -> 346; 128^2
+// over 128^3 at S = 256 69 -> 23 and 112 -> 30; 64^2 over 64^3 at S = 128
+// forward 37 -> 12.
+constexpr int kSplitWaves = 8, kSplitRun = 4, kSplitRound = (kSplitWaves - 1) * kSplitRun;
+
+// Wave tile of this workgroup; P's walk is that of the wave tiles.
+__device__ __forceinline__ bool split_tile(const Params &P, int &view, int &row, int &col, int &wslot) {
+    wslot = tile_index(P);
+    if (wslot >= P.total_tiles) return false;
+    view = wslot / P.wt_per_view;
+    const int r = wslot - view * P.wt_per_view, wy = r / P.wt_x, wx = r - wy * P.wt_x, lane = threadIdx.x & 63;
+    row = P.bundle ? 0 : wy * 8 + (lane >> 3);
+    col = P.bundle ? wx * 64 + lane : wx * 8 + (lane & 7);
+    return true;
+}
+
+// One run of samples [k0, k0 + kSplitRun) of the lane's ray: emit(j, value,
+// slopes).  An outside sample has zero slopes and the value `none`.
+template <typename T, int LAYOUT, bool SLOPES, bool INTERIOR, typename F>
+__device__ __forceinline__ void split_run(const Params &P, const T *field, const float *o, const float *d, float lower,
+                                          float step, int k0, bool checked, float none, F emit) {
+    float v[kSplitRun][8];
+    Cell32 c[kSplitRun];
+    bool in[kSplitRun], fresh[kSplitRun];
+#pragma unroll
+    for (int j = 0; j < kSplitRun; ++j) {
+        const float pos = fmaf(sample_centre(P, min(k0 + j, P.samples - 1)), step, lower);
+        const float p0 = fmaf(pos, d[0], o[0]);
+        const float p1 = fmaf(pos, d[1], o[1]);
+        const float p2 = fmaf(pos, d[2], o[2]);
+        if constexpr (INTERIOR)
+            cell32_interior(P, p0, p1, p2, c[j]);
+        else
+            cell32_inside(P, p0, p1, p2, c[j]);  // clamped: the load stays in the field
+        in[j] = INTERIOR || !checked || inside32(P, p0, p1, p2);
+        // only lanes whose cell changed load: requests to the L2 bound the march
+        fresh[j] = j == 0 || c[j].base != c[j > 0 ? j - 1 : 0].base;
+        if (fresh[j]) load8<T, LAYOUT>(P, field, c[j].base, v[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < kSplitRun; ++j) {
+        if (j > 0) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[j][q] = fresh[j] ? v[j][q] : v[j > 0 ? j - 1 : 0][q];
+        }
+        float wt[8], g[3] = {0.0f, 0.0f, 0.0f};
+        weights32(c[j], wt);
+        const float value = interpolate32(wt, v[j]);
+        if constexpr (SLOPES) {
+            slopes32(c[j], v[j], g);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) g[a] = in[j] ? g[a] : 0.0f;
+        }
+        emit(j, in[j] ? value : none, g);
+    }
+}
+
+template <typename T, bool COMPENSATED, int LAYOUT>
+__global__ __launch_bounds__(64 * kSplitWaves) void forward32_split_kernel(Params P, const T *__restrict__ field,
+                                                                           float *__restrict__ out) {
+    __shared__ float buffer[2][kSplitRound][64];
+    int view, row, col, wslot;
+    if (!split_tile(P, view, row, col, wslot)) return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool adds = w == kSplitWaves - 1;
+    const bool exists = ray_in_range(P, view, row, col);
+    bool hit = false;
+    float o[3] = {0, 0, 0}, d[3] = {0, 0, 0}, len = 0.0f, lower = 0.0f, step = 0.0f;
+    if (exists) {
+        World ww;
+        ray_world(P, P.poses + 12 * (size_t)view, view, row, col, ww);
+        Ray r;
+        ray_grid(P, ww, r);
+        const float ro[3] = {(float)r.o[0], (float)r.o[1], (float)r.o[2]};
+        const float rd[3] = {(float)r.d[0], (float)r.d[1], (float)r.d[2]};
+        len = (float)r.len;
+        if (!r.valid || !finite3f(ro[0], ro[1], ro[2]) || !finite3f(rd[0], rd[1], rd[2]) || !isfinite(len) ||
+            len <= 0.0f) {
+            if (adds) flag(P, view, DPT_STATUS_RANGE);
+        } else {
+            const Interval32 iv = interval32(P, ro, rd);
+            if (iv.upper > iv.lower) {
+                lower = iv.lower;
+                step = (iv.upper - iv.lower) / (float)P.samples;
+                // a ray with non-finite sample points keeps the benign ray
+                // (its image is flagged)
+                hit = finite_span(ro, rd, lower, step, 0, P.samples);
+                if (!hit && adds) flag(P, view, DPT_STATUS_RANGE);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    o[a] = hit ? ro[a] : 0.0f;
+                    d[a] = hit ? rd[a] : 0.0f;
+                }
+                if (!hit) lower = step = 0.0f;
+            }
+        }
+    }
+    float result = 0.0f;
+    if (__builtin_amdgcn_ballot_w64(hit) != 0) {  // the same in every wave
+        const bool checked = __builtin_amdgcn_ballot_w64(hit && !span_inside(P, o, d, lower, step, 0, P.samples)) != 0;
+        int ka = P.samples, kb = P.samples;
+        if (hit) interior_span(P, o, d, lower, step, 0, P.samples, ka, kb);
+        // lanes without a hit sample the origin, an interior point on grids with cells on every axis
+        const bool origin = interior32(P, 0.0f, 0.0f, 0.0f);
+        const int first_hit = __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(hit)) - 1;
+        ka = __builtin_amdgcn_readlane(ka, first_hit);
+        kb = origin ? __builtin_amdgcn_readlane(kb, first_hit) : ka;
+        Acc<COMPENSATED> total;
+        total.init();
+        const int rounds = (P.samples + kSplitRound - 1) / kSplitRound;
+        for (int r = 0; r <= rounds; ++r) {
+            if (!adds) {
+                const int k0 = r * kSplitRound + w * kSplitRun;
+                if (k0 < P.samples) {
+                    float(*slot)[64] = &buffer[r & 1][w * kSplitRun];
+                    auto emit = [&](int j, float value, const float *) { slot[j][lane] = value; };
+                    // -0 is the identity of FP32 addition (the reference skips outside samples)
+                    if (k0 >= ka && k0 + kSplitRun <= kb)
+                        split_run<T, LAYOUT, false, true>(P, field, o, d, lower, step, k0, false, -0.0f, emit);
+                    else
+                        split_run<T, LAYOUT, false, false>(P, field, o, d, lower, step, k0, checked, -0.0f, emit);
+                }
+            } else if (r > 0) {
+                const int base = (r - 1) * kSplitRound, count = min(kSplitRound, P.samples - base);
+                const float(*slot)[64] = buffer[(r - 1) & 1];
+                auto add = [&](int k, float value) {
+                    if constexpr (COMPENSATED) {
+                        if (k > 0 && (k % kFoldBlock) == 0) total.fold();
+                    }
+                    total.add(value);
+                };
+                if (count == kSplitRound) {  // every read in flight before the first addition
+                    float e[kSplitRound];
+#pragma unroll
+                    for (int s = 0; s < kSplitRound; ++s) e[s] = slot[s][lane];
+#pragma unroll
+                    for (int s = 0; s < kSplitRound; ++s) add(base + s, e[s]);
+                } else {
+                    for (int s = 0; s < count; ++s) add(base + s, slot[s][lane]);
+                }
+            }
+            __syncthreads();
+        }
+        if (hit) result = total.value() * (len * step);
+    }
+    if (adds && exists) {
+        const size_t ray = ((size_t)view * P.rows + row) * P.cols + col;
+        out[ray] = result;
+        if (!isfinite(result)) flag(P, view, DPT_STATUS_RANGE);
+    }
+}
+
+template <typename T, int C, bool COMPENSATED, int LAYOUT>
+__global__ __launch_bounds__(64 * kSplitWaves) void vjp32_split_kernel(Params P, const T *__restrict__ field,
+                                                                       const float *__restrict__ seeds,
+                                                                       double *__restrict__ partials) {
+    __shared__ float4 buffer[2][kSplitRound][64];
+    int view, row, col, wslot;
+    if (!split_tile(P, view, row, col, wslot)) return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool adds = w == kSplitWaves - 1;
+    const double *pose = P.poses + 12 * (size_t)view;
+    bool active = false;
+    float o[3] = {0, 0, 0}, d[3] = {0, 0, 0}, len = 0.0f, seed = 0.0f, span = 0.0f, lower = 0.0f, step = 0.0f;
+    Interval32 iv{};
+    if (ray_in_range(P, view, row, col)) {
+        World ww;
+        ray_world(P, pose, view, row, col, ww);
+        Ray r;
+        ray_grid(P, ww, r);
+        const float ro[3] = {(float)r.o[0], (float)r.o[1], (float)r.o[2]};
+        const float rd[3] = {(float)r.d[0], (float)r.d[1], (float)r.d[2]};
+        len = (float)r.len;
+        if (!r.valid || !finite3f(ro[0], ro[1], ro[2]) || !finite3f(rd[0], rd[1], rd[2]) || !isfinite(len) ||
+            len <= 0.0f) {
+            if (adds) flag(P, view, DPT_STATUS_RANGE);
+        } else {
+            iv = interval32(P, ro, rd);
+            span = iv.upper - iv.lower;
+            seed = seeds[((size_t)view * P.rows + row) * P.cols + col];
+            if (!isfinite(seed) && adds) flag(P, view, DPT_STATUS_RANGE);
+            if (span > 0.0f && seed != 0.0f) {
+                lower = iv.lower;
+                step = span / (float)P.samples;
+                // a ray with non-finite sample points is flagged and adds nothing
+                active = finite_span(ro, rd, lower, step, 0, P.samples);
+                if (!active && adds) flag(P, view, DPT_STATUS_RANGE);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    o[a] = active ? ro[a] : 0.0f;
+                    d[a] = active ? rd[a] : 0.0f;
+                }
+                if (!active) lower = step = 0.0f;
+            }
+        }
+    }
+    PoseSums<COMPENSATED> q;
+    q.init();
+    if (__builtin_amdgcn_ballot_w64(active) != 0) {  // the same in every wave
+        const bool checked = __builtin_amdgcn_ballot_w64(active && !span_inside(P, o, d, lower, step, 0, P.samples)) != 0;
+        int ka = P.samples, kb = P.samples;
+        if (active) interior_span(P, o, d, lower, step, 0, P.samples, ka, kb);
+        const bool origin = interior32(P, 0.0f, 0.0f, 0.0f);  // as forward32_split_kernel
+        const int first_hit = __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(active)) - 1;
+        ka = __builtin_amdgcn_readlane(ka, first_hit);
+        kb = origin ? __builtin_amdgcn_readlane(kb, first_hit) : ka;
+        const int rounds = (P.samples + kSplitRound - 1) / kSplitRound;
+        for (int r = 0; r <= rounds; ++r) {
+            if (!adds) {
+                const int k0 = r * kSplitRound + w * kSplitRun;
+                if (k0 < P.samples) {
+                    float4(*slot)[64] = &buffer[r & 1][w * kSplitRun];
+                    auto emit = [&](int j, float value, const float *g) {
+                        slot[j][lane] = make_float4(value, g[0], g[1], g[2]);
+                    };
+                    if (k0 >= ka && k0 + kSplitRun <= kb)
+                        split_run<T, LAYOUT, true, true>(P, field, o, d, lower, step, k0, false, 0.0f, emit);
+                    else
+                        split_run<T, LAYOUT, true, false>(P, field, o, d, lower, step, k0, checked, 0.0f, emit);
+                }
+            } else if (r > 0) {
+                const int base = (r - 1) * kSplitRound, count = min(kSplitRound, P.samples - base);
+                const float4(*slot)[64] = buffer[(r - 1) & 1];
+                auto add = [&](int k, const float4 &e) {
+                    if constexpr (COMPENSATED) {
+                        if (k > 0 && (k % kFoldBlock) == 0) q.fold();
+                    }
+                    q.add(P, k, fmaf(sample_centre(P, k), step, lower), e.x, e.y, e.z, e.w, d);
+                };
+                if (count == kSplitRound) {  // reads in flight, a wave's share at a time
+                    constexpr int kPart = kSplitRound / 2;
+#pragma unroll
+                    for (int part = 0; part < 2; ++part) {
+                        float4 e[kPart];
+#pragma unroll
+                        for (int s = 0; s < kPart; ++s) e[s] = slot[part * kPart + s][lane];
+#pragma unroll
+                        for (int s = 0; s < kPart; ++s) add(base + part * kPart + s, e[s]);
+                    }
+                } else {
+                    for (int s = 0; s < count; ++s) add(base + s, slot[s][lane]);
+                }
+            }
+            __syncthreads();
+        }
+    }
+    if (adds)
+        pose_finish<C, COMPENSATED>(P, pose, active, q, iv, len, seed, span, step, partials, wslot, true, view, row,
+                                    col);
 }
 
 // --------------------------------------------------------- FP64 sampling --
@@ -1651,8 +1795,7 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
     const double *pose = P.poses + 12 * (size_t)view;
     int first = 0, last = P.samples;
     if (P.segments > 1) {
-        const int b = blockIdx.x;
-        const int seg = ((b % kXcds) * P.chunk + b / kXcds) / P.base_tiles;
+        const int seg = tile_index(P) / P.base_tiles;
         first = seg * P.segment_samples;
         last = min(first + P.segment_samples, P.samples);
     }
@@ -2161,7 +2304,6 @@ struct dpt_plan {
     int *d_status = nullptr;
     int32_t *h_status = nullptr;
     double *d_partials = nullptr;
-    int partial_segments = 1;              // d_partials holds this many segments' wave partials
     double *d_acc = nullptr;
     float *d_alpha = nullptr;
     double *d_alpha64 = nullptr;
@@ -2219,6 +2361,16 @@ unsigned grid_blocks(int64_t n) {
     return (unsigned)b;
 }
 
+// XCD walk of a launch (walk_index): rows of tiles in turn for few views with
+// rows for every XCD, else contiguous runs.
+constexpr int kFewViews = 2 * kXcds;
+bool rows_in_turn(int views, int rows) { return views < kFewViews && rows >= 2 * kXcds; }
+void set_walk(Params &P) {
+    const int rows = P.total_tiles / P.tiles_x;
+    P.by_rows = rows_in_turn(P.views, rows);
+    P.chunk = P.by_rows ? (rows + kXcds - 1) / kXcds * P.tiles_x : (P.total_tiles + kXcds - 1) / kXcds;
+}
+
 // Tile geometry for `vb` views per workgroup (see lane_ray).
 void configure_tiles(Params &P, int vb) {
     P.vb = P.bundle ? 1 : vb;
@@ -2238,26 +2390,21 @@ void configure_tiles(Params &P, int vb) {
     P.tiles_y = (P.rows + P.tile_h - 1) / P.tile_h;
     P.tiles_per_group = P.tiles_x * P.tiles_y;
     P.total_tiles = P.tiles_per_group * ((P.views + P.vb - 1) / P.vb);
-    P.chunk = (P.total_tiles + kXcds - 1) / kXcds;
+    set_walk(P);
     P.segments = 1;
     P.base_tiles = P.total_tiles;
     P.segment_samples = P.samples;
 }
 
-// Sample-range segments of the FP32 VJP: a launch of few tiles (one view of
-// 512^2 is 1024 workgroups, one wave per SIMD) leaves every wave walking all
-// its samples with its memory latency exposed.  Such launches run each tile
-// as `segments` workgroups over consecutive ranges of whole chunks (at least
-// two chunks and 256 samples each), aiming at 16384 waves; the pose partials
-// of a ray's segments are summed in FP64 by the fixed-order reduction, the
-// volume increments of each segment go to the brick as before.  A segmented
-// pose gradient is not the reference's one sequential FP32 sum per ray, so
-// only 16-bit storage (blocked compensated sums, no FP32 counterpart)
-// segments the pose; FP32 storage runs it unsegmented in the pipelined loop.
-// DPT_AMD_VJP_SEGMENTS overrides the count (1..8; not the two-chunk floor).
+// Sample-range segments of the volume adjoint: a launch of few tiles (one view
+// of 512^2 is 1024 workgroups, one wave per SIMD) runs each tile as `segments`
+// workgroups over consecutive ranges of whole chunks (at least two chunks and
+// 256 samples each), aiming at 16384 waves.  DPT_AMD_VJP_SEGMENTS overrides
+// the count (1..8; not the two-chunk floor).
 // A launch of at most 8192 waves (8 per SIMD): one whose sample loops expose
 // their memory latency.
-bool small_launch(const Params &P) { return (long long)P.total_tiles * (kBlock / 64) * 2 <= 16384; }
+// (7 views of 257 x 301, 9064 waves, run 7 % slower split.)
+bool small_launch(const Params &P) { return (long long)P.total_tiles * (kBlock / 64) <= 8192; }
 
 void configure_segments(Params &P) {
     const long long waves = (long long)P.total_tiles * (kBlock / 64);
@@ -2277,7 +2424,7 @@ void configure_segments(Params &P) {
     P.segment_samples = per * P.chunk_samples;
     P.base_tiles = P.total_tiles;
     P.total_tiles = P.base_tiles * g;
-    P.chunk = (P.total_tiles + kXcds - 1) / kXcds;
+    set_walk(P);
 }
 
 // Views share a workgroup (and its LDS brick) only when their central rays
@@ -2390,6 +2537,13 @@ Params launch_params(const dpt_plan *p, const double *poses) {
 }
 
 unsigned tile_grid(const Params &P) { return (unsigned)(P.chunk * kXcds); }
+// One workgroup per wave tile (split_tile).
+Params split_params(Params P) {
+    P.tiles_x = P.wt_x;
+    P.total_tiles = P.views * P.wt_per_view;
+    set_walk(P);
+    return P;
+}
 
 // Launch parameters of a gather from the plan's copy (quads or cells).
 Params copy_params(const dpt_plan *p, Params P) {
@@ -2406,19 +2560,18 @@ int launch_forward(dpt_plan *p, const Params &P, const void *field, void *out, b
     if (p->arithmetic == DPT_ARITH_FP32) {
         float *o = static_cast<float *>(out);
         constexpr bool HALF = !std::is_same<T, float>::value;
-        if constexpr (!HALF) {
-            if (small_launch(P)) {
-                if (cells)
-                    hipLaunchKernelGGL((forward32_kernel<T, false, kGatherCopy<T>, true>), grid, block, 0, s,
-                                       copy_params(p, P), static_cast<const T *>(p->d_copy), o);
-                else if (P.nx > 1)
-                    hipLaunchKernelGGL((forward32_kernel<T, false, kLayoutPair, true>), grid, block, 0, s, P, f, o);
-                else
-                    hipLaunchKernelGGL((forward32_kernel<T, false, kLayoutScalar, true>), grid, block, 0, s, P, f,
-                                       o);
-                HIP_TRY(hipGetLastError());
-                return DPT_OK;
-            }
+        if (small_launch(P)) {
+            const Params Q = split_params(P);
+            const dim3 tiles(tile_grid(Q)), lanes(64 * kSplitWaves);
+            if (cells)
+                hipLaunchKernelGGL((forward32_split_kernel<T, HALF, kGatherCopy<T>>), tiles, lanes, 0, s,
+                                   copy_params(p, Q), static_cast<const T *>(p->d_copy), o);
+            else if (P.nx > 1)
+                hipLaunchKernelGGL((forward32_split_kernel<T, HALF, kLayoutPair>), tiles, lanes, 0, s, Q, f, o);
+            else
+                hipLaunchKernelGGL((forward32_split_kernel<T, HALF, kLayoutScalar>), tiles, lanes, 0, s, Q, f, o);
+            HIP_TRY(hipGetLastError());
+            return DPT_OK;
         }
         if (cells)
             hipLaunchKernelGGL((forward32_kernel<T, HALF, kGatherCopy<T>>), grid, block, 0, s, copy_params(p, P),
@@ -2444,34 +2597,34 @@ double *pose_destination(dpt_plan *p) {
 }
 
 template <typename T, int C, int LAYOUT>
-void launch_vjp32(dpt_plan *p, const Params &P, const T *f, const float *sd, bool pipe, hipStream_t s) {
+void launch_vjp32(dpt_plan *p, const Params &P, const T *f, const float *sd, hipStream_t s) {
     constexpr bool HALF = !std::is_same<T, float>::value;
-    const dim3 grid(tile_grid(P)), block(kBlock);
     double *partials = pose_destination<C>(p);
-    if constexpr (!HALF && (C == 6 || C == 12)) {
-        if (pipe) {
-            hipLaunchKernelGGL((vjp32_kernel<T, C, false, LAYOUT, true>), grid, block, 0, s, P, f, sd, partials);
-            return;
-        }
+    if (small_launch(P)) {
+        const Params Q = split_params(P);
+        hipLaunchKernelGGL((vjp32_split_kernel<T, C, HALF, LAYOUT>), dim3(tile_grid(Q)), dim3(64 * kSplitWaves), 0, s,
+                           Q, f, sd, partials);
+    } else {
+        hipLaunchKernelGGL((vjp32_kernel<T, C, HALF, LAYOUT>), dim3(tile_grid(P)), dim3(kBlock), 0, s, P, f, sd,
+                           partials);
     }
-    hipLaunchKernelGGL((vjp32_kernel<T, C, HALF, LAYOUT>), grid, block, 0, s, P, f, sd, partials);
 }
 
 // Pose adjoint of a midpoint plan, or the joint adjoint of a cell-Gauss plan.
 template <typename T, int C>
 int launch_vjp_c(dpt_plan *p, const Params &P, const void *field, const void *seeds, bool vol, bool pose,
-                 bool cells, hipStream_t s, bool pipe = false) {
+                 bool cells, hipStream_t s) {
     const T *f = static_cast<const T *>(field);
     const dim3 grid(tile_grid(P)), block(kBlock);
     double *partials = pose_destination<C>(p);
     if (p->arithmetic == DPT_ARITH_FP32) {
         const float *sd = static_cast<const float *>(seeds);
         if (cells && P.nx > 1)
-            launch_vjp32<T, C, kGatherCopy<T>>(p, copy_params(p, P), static_cast<const T *>(p->d_copy), sd, pipe, s);
+            launch_vjp32<T, C, kGatherCopy<T>>(p, copy_params(p, P), static_cast<const T *>(p->d_copy), sd, s);
         else if (P.nx > 1)
-            launch_vjp32<T, C, kLayoutPair>(p, P, f, sd, pipe, s);
+            launch_vjp32<T, C, kLayoutPair>(p, P, f, sd, s);
         else
-            launch_vjp32<T, C, kLayoutScalar>(p, P, f, sd, pipe, s);
+            launch_vjp32<T, C, kLayoutScalar>(p, P, f, sd, s);
     } else {
         const double *sd = static_cast<const double *>(seeds);
         const size_t lds = (size_t)P.brick_cap * sizeof(double);
@@ -2493,11 +2646,11 @@ int launch_vjp_c(dpt_plan *p, const Params &P, const void *field, const void *se
 
 template <typename T>
 int launch_vjp(dpt_plan *p, const Params &P, const void *field, const void *seeds, bool vol, bool pose,
-               int components, bool cells, hipStream_t s, bool pipe = false) {
+               int components, bool cells, hipStream_t s) {
     if (components == kRayCoordinates) return launch_vjp_c<T, kRayCoordinates>(p, P, field, seeds, false, true, cells, s);
     if (components == kRayTangent) return launch_vjp_c<T, kRayTangent>(p, P, field, seeds, false, true, cells, s);
-    if (components == 6) return launch_vjp_c<T, 6>(p, P, field, seeds, vol, pose, cells, s, pipe);
-    return launch_vjp_c<T, 12>(p, P, field, seeds, vol, pose, cells, s, pipe);
+    if (components == 6) return launch_vjp_c<T, 6>(p, P, field, seeds, vol, pose, cells, s);
+    return launch_vjp_c<T, 12>(p, P, field, seeds, vol, pose, cells, s);
 }
 
 int launch_walk(dpt_plan *p, const Params &P, const void *seeds, hipStream_t s) {
@@ -2873,23 +3026,7 @@ int dpt_vjp(dpt_plan *p, const void *field, const double *poses, const void *cot
     P.volume_f64 = vol64 ? 1 : 0;
     configure_tiles(P, p->vjp_vb);
     const Params whole = P;
-    if (p->arithmetic == DPT_ARITH_FP32 && !p->cell_gauss) configure_segments(P);
-    // FP32 storage keeps each ray's pose sums one sequential FP32 sum, as the
-    // reference: a segmented launch takes the pose unsegmented through the
-    // pipelined loop, beside a segmented volume-only launch
-    const bool pipe = pose && P.segments > 1 && p->storage == DPT_STORE_F32;
-    const int pose_segments = pipe ? 1 : P.segments;
-    if (pose && pose_segments > p->partial_segments) {
-        // grown once per plan, for launches small enough to take segments
-        HIP_TRY(hipStreamSynchronize(s));
-        (void)hipFree(p->d_partials);
-        p->d_partials = nullptr;
-        p->partial_segments = 0;
-        if (hipMalloc((void **)&p->d_partials,
-                      sizeof(double) * kMaxComponents * (size_t)P.wt_per_view * P.views * pose_segments) != hipSuccess)
-            return fail(DPT_E_MEMORY, "pose partials allocation failed");
-        p->partial_segments = pose_segments;
-    }
+    if (vol && !p->cell_gauss) configure_segments(P);  // of the volume adjoint
     if (!(flags & DPT_NO_CHECKS)) {
         switch (p->storage) {
         case DPT_STORE_F32:
@@ -2930,12 +3067,11 @@ int dpt_vjp(dpt_plan *p, const void *field, const double *poses, const void *cot
     if (walk) rc = launch_walk(p, P, cotangent, s);
     if (rc == DPT_OK && (pose || !walk)) {
         if (p->storage == DPT_STORE_F32)
-            rc = launch_vjp<float>(p, pose_segments == 1 ? whole : P, field, cotangent, vol, pose, components, cells, s,
-                                   pipe);
+            rc = launch_vjp<float>(p, whole, field, cotangent, vol, pose, components, cells, s);
         else if (p->storage == DPT_STORE_BF16)
-            rc = launch_vjp<__hip_bfloat16>(p, P, field, cotangent, vol, pose, components, cells, s);
+            rc = launch_vjp<__hip_bfloat16>(p, whole, field, cotangent, vol, pose, components, cells, s);
         else
-            rc = launch_vjp<__half>(p, P, field, cotangent, vol, pose, components, cells, s);
+            rc = launch_vjp<__half>(p, whole, field, cotangent, vol, pose, components, cells, s);
     }
     timer_end(p, 1, s);
     if (rc != DPT_OK) return rc;
@@ -2943,10 +3079,10 @@ int dpt_vjp(dpt_plan *p, const void *field, const double *poses, const void *cot
     if (pose) {
         if (components == 6)
             hipLaunchKernelGGL(pose_reduce_kernel<6>, dim3(P.views), dim3(kBlock), 0, s, p->d_partials,
-                               pose_segments * P.wt_per_view, grad_pose, accumulate, p->d_status);
+                               P.wt_per_view, grad_pose, accumulate, p->d_status);
         else
             hipLaunchKernelGGL(pose_reduce_kernel<12>, dim3(P.views), dim3(kBlock), 0, s, p->d_partials,
-                               pose_segments * P.wt_per_view, grad_pose, accumulate, p->d_status);
+                               P.wt_per_view, grad_pose, accumulate, p->d_status);
     }
     if (vol64)
         hipLaunchKernelGGL(finish_volume_kernel<double>, dim3(grid_blocks(p->voxels)), dim3(kBlock), 0, s,
