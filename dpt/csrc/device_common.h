@@ -52,11 +52,11 @@ struct Params {
     const double *ray_end;
     const double *poses;     // views x 12
     int *status;             // views
-    int brick_cap;           // FP64 LDS brick entries per workgroup of the cell-Gauss volume adjoint
-    int walk_cap;            // FP64 LDS brick entries per workgroup of the midpoint volume adjoint
+    int brick_cap;           // index-chunk brick estimate of the plan (choose_brick_cap)
+    int walk_cap;            // FP64 LDS brick entries per workgroup of the volume adjoint
     int slab_chunks;         // 1: index chunks would overflow even the larger brick often (silhouette-heavy plans)
     int chunk_samples;       // unit of the sample segments
-    int gauss_chunks;        // lockstep chunks per ray of the cell-Gauss volume adjoint
+    int gauss_chunks;        // first slabs per axis of the cell-Gauss volume adjoint
     const double *alpha64;   // 2 x samples entries (FP64 sampling): (k + 0.5) / S, then 1 - that
     const float *alpha;      // 3 x samples entries: alpha_k, k + 0.5, 1 - alpha_k (sample_table_entries)
     int volume_f64;          // 1: FP64 volume destination (increments unflushed, FP64 sampling unrounded)

@@ -18,6 +18,8 @@ torch = pytest.importorskip("torch")
 
 pytestmark = pytest.mark.gpu
 
+from dpt import _native  # noqa: E402
+
 from .test_gpu_parity import NativeScene, _rel  # noqa: E402
 
 
@@ -84,3 +86,22 @@ def test_more_samples_than_the_float_counter_holds():
     rays = (np.array([[-4.0, 0.3, 0.9]]), np.array([[7.0, 1.4, 1.6]]))
     actual, expected = _volume(grid, 5_000_000, "float32", rays=rays)
     assert _rel(actual, expected) <= 1e-5
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-33])
+@pytest.mark.parametrize("shape", [(24, 26, 28), (1, 26, 28), (24, 26, 1)])
+def test_cell_gauss_pieces_match_the_oracle(shape, scale):
+    """Factors in the walk's range, and below 2^-102, whose rays take the
+    reference's products piece by piece."""
+    print(f"case walk gauss {shape} {scale}", flush=True)
+    grid = O.Grid(shape, (1.0, 0.9, 1.1), tuple(-0.5 * (n - 1) * h for n, h in zip(shape[::-1], (1.0, 0.9, 1.1))))
+    panels = scenes.cone_panels(grid, 3, 19, 21, sod=120.0, sdd=200.0, offset=0.3)
+    seeds = scale * np.random.default_rng(2).uniform(-1.0, 1.0, 3 * 19 * 21)
+    values = np.full(grid.voxels, 0.02, dtype=np.float32)
+    expected, _, _, _ = O.Scene(grid, 7, panels=panels).vjp(values, seeds, precision="fp64", pose=False,
+                                                           integration="cell_gauss")
+    gpu = NativeScene(grid, 7, panels=panels, precision="float64", extra_needs=_native.CELL_GAUSS)
+    actual, _, status = gpu.vjp(values, seeds, pose_grad=False)
+    assert not any(status)
+    # FP32-rounded increments, then one FP32 rounding of each sum
+    assert _rel(actual / scale, expected / scale) <= 1e-7
