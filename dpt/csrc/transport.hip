@@ -8,8 +8,8 @@
 // (seed, history identity) alone, whatever thread or order runs it.
 //
 // trace_kernel: persistent grid.  Each wave keeps 64 photons in flight and
-//   refills a lane as soon as its photon terminates (history regeneration):
-//   the wave grabs identities in chunks of 256 from a device counter, and new
+//   refills lanes whose photons terminated (history regeneration) once kRefill
+//   of them wait: the wave grabs identities in chunks of 256 from a device counter, and new
 //   photons are ranked over the idle lanes with a ballot.  Lanes therefore do
 //   not idle behind the longest history of a fixed batch.  The material and
 //   interaction tables (a few KB) are staged once per workgroup in LDS; the
@@ -680,10 +680,16 @@ __device__ __forceinline__ void finish_rayleigh(Photon &ph, const Angular &r) {
 
 __global__ void zero_counter_kernel(unsigned long long *counter) { *counter = 0ull; }
 
-// WAVES: minimum waves per SIMD the register allocation must allow (2 fits
-// the whole walk in registers; 4 trades a few spills for occupancy).
-template <int WAVES>
-__global__ __launch_bounds__(kBlock, WAVES) void trace_kernel(Model m, Call c) {
+// Lanes that wait for an ended photon's score or a new photon before the wave
+// stops for them.  A wave ran both at every event, for one lane in twelve:
+// 10^7 histories of the 40-120 keV spectrum on 128^3 take 7.29 / 7.04 / 6.54 /
+// 6.48 / 6.66 ms at 1 / 8 / 16 / 24 / 32.
+constexpr int kRefill = 20;
+
+// Three waves per SIMD: 168 VGPRs and 112 bytes of spills.  Four spill 264
+// bytes, whose traffic ran to 3.7 TB/s (7.07 ms against 6.54); two leave the
+// divergent FP64 chains exposed (7.31).
+__global__ __launch_bounds__(kBlock, 3) void trace_kernel(Model m, Call c) {
     extern __shared__ double lds[];
     __shared__ unsigned int hist[8];
     for (int i = threadIdx.x; i < m.table_doubles; i += kBlock) lds[i] = c.tables[i];
@@ -698,43 +704,13 @@ __global__ __launch_bounds__(kBlock, WAVES) void trace_kernel(Model m, Call c) {
     Photon ph;
     ph.alive = false;
     for (;;) {
-        // Refill idle lanes from this wave's queue of history identities.
-        uint64_t need = __ballot(!has);
-        while (need != 0ull && !exhausted) {
-            if (q_next >= q_end) {
-                unsigned long long base = 0ull;
-                if (lane == 0) base = atomicAdd(c.counter, (unsigned long long)kChunk);
-                base = __shfl(base, 0);
-                if (base >= count) {
-                    exhausted = true;
-                    break;
-                }
-                q_next = base;
-                q_end = min(base + kChunk, count);
-            }
-            const uint64_t avail = q_end - q_next;
-            const uint64_t rank = (uint64_t)__popcll(need & below);
-            if (!has && rank < avail) {
-                start(m, c, T, c.first + q_next + rank, ph);
-                has = true;
-            }
-            q_next += min((uint64_t)__popcll(need), avail);
-            need = __ballot(!has);
-        }
-        if (__ballot(has) == 0ull) break;
-        PendingRayleigh pend{false, 0, 0u};
-        if (has && ph.alive) event_step(m, c, T, ph, pend);
-        // Rayleigh draws, one photon at a time by the whole wave (all lanes
-        // active here; the loop bound and the leader's values are uniform)
-        for (uint64_t waiting = __ballot(pend.pending); waiting != 0ull; waiting &= waiting - 1ull) {
-            const int leader = __ffsll((unsigned long long)waiting) - 1;
-            const Angular r = rayleigh_event_wave(m, T, __shfl(ph.energy, leader, 64), __shfl(pend.material, leader, 64),
-                                                  c.seed, __shfl(ph.history, leader, 64),
-                                                  (uint32_t)__shfl((int)pend.event, leader, 64), lane);
-            if (lane == leader) finish_rayleigh(ph, r);
-        }
-        if (has) {
-            if (!ph.alive) {
+        // Photons that ended and empty lanes are served together once
+        // kRefill lanes wait (or no photon is in flight): ending and starting
+        // a photon cost as much as an event and would otherwise run at
+        // every event for the few lanes that need them.
+        const uint64_t idle = __ballot(!has || !ph.alive);
+        if (__popcll(idle) >= kRefill || idle == ~0ull) {
+            if (has && !ph.alive) {
                 // Termination: detector hit and score (transport/kernels.py:1520-1536).
                 int pixel = kMissPixel;
                 double score = 0.0;
@@ -764,6 +740,41 @@ __global__ __launch_bounds__(kBlock, WAVES) void trace_kernel(Model m, Call c) {
                 if (ph.status >= EVENT_BUDGET) atomicOr(c.failure_bits, 1 << ph.status);
                 has = false;
             }
+            // Refill idle lanes from this wave's queue of history identities.
+            uint64_t need = __ballot(!has);
+            while (need != 0ull && !exhausted) {
+                if (q_next >= q_end) {
+                    unsigned long long base = 0ull;
+                    if (lane == 0) base = atomicAdd(c.counter, (unsigned long long)kChunk);
+                    base = __shfl(base, 0);
+                    if (base >= count) {
+                        exhausted = true;
+                        break;
+                    }
+                    q_next = base;
+                    q_end = min(base + kChunk, count);
+                }
+                const uint64_t avail = q_end - q_next;
+                const uint64_t rank = (uint64_t)__popcll(need & below);
+                if (!has && rank < avail) {
+                    start(m, c, T, c.first + q_next + rank, ph);
+                    has = true;
+                }
+                q_next += min((uint64_t)__popcll(need), avail);
+                need = __ballot(!has);
+            }
+            if (__ballot(has) == 0ull) break;
+        }
+        PendingRayleigh pend{false, 0, 0u};
+        if (has && ph.alive) event_step(m, c, T, ph, pend);
+        // Rayleigh draws, one photon at a time by the whole wave (all lanes
+        // active here; the loop bound and the leader's values are uniform)
+        for (uint64_t waiting = __ballot(pend.pending); waiting != 0ull; waiting &= waiting - 1ull) {
+            const int leader = __ffsll((unsigned long long)waiting) - 1;
+            const Angular r = rayleigh_event_wave(m, T, __shfl(ph.energy, leader, 64), __shfl(pend.material, leader, 64),
+                                                  c.seed, __shfl(ph.history, leader, 64),
+                                                  (uint32_t)__shfl((int)pend.event, leader, 64), lane);
+            if (lane == leader) finish_rayleigh(ph, r);
         }
     }
     __syncthreads();
@@ -801,8 +812,7 @@ struct dpt_transport {
     unsigned long long *d_histogram;
     int *d_bits;
     unsigned long long *h_histogram;  // pinned: 7 counts + bits
-    int grid2, grid4;
-    int waves;  // 2 or 4: trace_kernel variant
+    int grid;   // workgroups that fill the device
 };
 
 namespace {
@@ -1011,16 +1021,12 @@ int dpt_transport_create(const dpt_transport_model *md, int32_t device, dpt_tran
         dpt_transport_destroy(t);
         return tr_fail(DPT_E_DEVICE, "device upload failed");
     }
-    int per_cu2 = 0, per_cu4 = 0, cus = 0;
+    int per_cu = 0, cus = 0;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) cus = prop.multiProcessorCount;
     const size_t lds = (size_t)m.table_doubles * sizeof(double);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu2, trace_kernel<2>, kBlock, lds) != hipSuccess) per_cu2 = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu4, trace_kernel<4>, kBlock, lds) != hipSuccess) per_cu4 = 0;
-    t->grid2 = std::max(1, per_cu2) * std::max(1, cus);
-    t->grid4 = std::max(1, per_cu4) * std::max(1, cus);
-    t->waves = 4;
-    if (const char *env = std::getenv("DPT_AMD_MC_WAVES")) t->waves = std::atoi(env) == 2 ? 2 : 4;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trace_kernel, kBlock, lds) != hipSuccess) per_cu = 0;
+    t->grid = std::max(1, per_cu) * std::max(1, cus);
     *out = t;
     return DPT_OK;
 }
@@ -1084,14 +1090,10 @@ int dpt_transport_trace(dpt_transport *t, const double *density, const dpt_point
     DeviceGuard guard(t->device);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t waves = (count + 63) / 64;
-    const int grid = t->waves == 2 ? t->grid2 : t->grid4;
-    const int blocks = (int)std::min<int64_t>(grid, (waves + 3) / 4);
+    const int blocks = (int)std::min<int64_t>(t->grid, (waves + 3) / 4);
     const size_t lds = (size_t)m.table_doubles * sizeof(double);
     zero_counter_kernel<<<1, 1, 0, s>>>(t->d_counter);
-    if (t->waves == 2)
-        trace_kernel<2><<<blocks, kBlock, lds, s>>>(m, c);
-    else
-        trace_kernel<4><<<blocks, kBlock, lds, s>>>(m, c);
+    trace_kernel<<<blocks, kBlock, lds, s>>>(m, c);
     if (hipGetLastError() != hipSuccess) return tr_fail(DPT_E_DEVICE, "trace launch failed");
     return DPT_OK;
 }
