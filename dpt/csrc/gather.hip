@@ -448,18 +448,31 @@ __device__ __forceinline__ GatherRay load_ray(const GatherRay *r) {
 //             running sum that starts at +0 is never -0).
 constexpr int kGeneral = 0, kSimple = 1, kMasked = 2;
 
+// The value of lane Q of each quad of lanes (DPP quad_perm).
+template <int Q>
+__device__ __forceinline__ double quad_lane(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), Q * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), Q * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
 // Add the contributions of ray g's samples k0..k1 to the voxel's total, in
 // sample then corner order (kernels/projection_adjoint.py:158-163 with
 // point_contribution, :33-44).
-template <int MODE, int MASK = 0>
+//
+// QUAD (kMasked): four neighbouring lanes hold one voxel, take four consecutive
+// samples a step and add the four addends in sample order, each broadcast
+// within the quad, so all four keep the same sum; a sample past k1 adds +0.
+template <int MODE, int MASK = 0, bool QUAD = false>
 __device__ __forceinline__ double add_ray(const Params &P, const GatherRay &g, const Voxel &vx, int k0, int k1,
                                           double total) {
     const int n[3] = {P.nx, P.ny, P.nz};
     const int cap[3] = {P.capx, P.capy, P.capz};
     const double vf = g.vf;
     if constexpr (MODE == kMasked) {
-        double kc = (double)k0 + 0.5;  // k + 0.5, exact
-        for (int k = k0; k <= k1; ++k, kc += 1.0) {
+        const int sub = QUAD ? (int)(threadIdx.x & 3) : 0;
+        double kc = (double)(k0 + sub) + 0.5;  // k + 0.5, exact
+        for (int k = k0; k <= k1; k += QUAD ? 4 : 1, kc += QUAD ? 4.0 : 1.0) {
             const double pos = g.lower + kc * g.step;
             double w[3];
 #pragma unroll
@@ -476,7 +489,16 @@ __device__ __forceinline__ double add_ray(const Params &P, const GatherRay &g, c
                     w[a] = !inside ? 0.0 : l == vx.i[a] ? 1.0 - f : l + 1 == vx.i[a] ? f : 0.0;
                 }
             }
-            total += ((vf * w[0]) * w[1]) * w[2];
+            const double addend = ((vf * w[0]) * w[1]) * w[2];
+            if constexpr (QUAD) {
+                const double own = k + sub <= k1 ? addend : 0.0;
+                total += quad_lane<0>(own);
+                total += quad_lane<1>(own);
+                total += quad_lane<2>(own);
+                total += quad_lane<3>(own);
+            } else {
+                total += addend;
+            }
         }
         return total;
     }
@@ -522,7 +544,7 @@ __device__ __forceinline__ double add_ray(const Params &P, const GatherRay &g, c
 }
 
 // The voxel's FP64 sum over every view, pixel window and sample window.
-template <int MODE, int MASK = 0>
+template <int MODE, int MASK = 0, bool QUAD = false>
 __device__ __forceinline__ double gather_voxel(const Params &P, const GatherRay *__restrict__ rays,
                                                const GatherView *__restrict__ views, const Voxel &vx) {
     const int64_t pixels = (int64_t)P.rows * P.cols;
@@ -554,7 +576,7 @@ __device__ __forceinline__ double gather_voxel(const Params &P, const GatherRay 
                 if (MODE == kMasked && !isfinite(g.vf))
                     total = add_ray<kSimple>(P, g, vx, k0, k1, total);
                 else
-                    total = add_ray<MODE, MASK>(P, g, vx, k0, k1, total);
+                    total = add_ray<MODE, MASK, QUAD>(P, g, vx, k0, k1, total);
             }
         }
     }
@@ -573,12 +595,18 @@ __device__ __forceinline__ double gather_voxel(const Params &P, const GatherRay 
 // The voxels along the grid's 12 edges (two coordinates within two samples
 // of a face) collect the most: every sample of every ray that clips that
 // edge, up to a hundred times an interior voxel.  They go before everything
-// else, each wave taking 64 consecutive voxels along one edge line: those
-// voxels' pixel windows advance through the same columns (or rows) in step,
-// so their long windows coincide in the wave instead of queueing one after
-// another.  The lanes of surface bricks that fall on an edge line are idle.
+// else, each wave taking 16 consecutive voxels along one edge line, a quad of
+// lanes to a voxel: those voxels' pixel windows advance through the same
+// columns (or rows) in step, so their long windows coincide in the wave
+// instead of queueing one after another, and the quad takes four samples a
+// step (24 views of 256^2 at S = 512 into 128^3: with a lane to a voxel the
+// edge waves ran up to 25 ms and the kernel 25.2; 15.5 with quads on the two
+// outermost samples, 8.6 with quads on four, next to which the rest runs 8).  The lanes of surface bricks that fall on an edge line are idle.
+constexpr int kEdgeVoxels = 16;  // voxels of an edge wave, a quad of lanes each
+
 struct BrickLayout {
     int edges;             // edge waves (0: no edge section, a grid axis below 4 samples)
+    int band;              // samples from a face that count as near it
     int zw, xw, yw;        // waves per edge line along z, x, y
     int edge_groups;       // workgroups of the edge section, a multiple of kXcds
     int nx, ny, nz;        // bricks per axis
@@ -591,14 +619,15 @@ struct BrickLayout {
 BrickLayout brick_layout(const Params &P) {
     BrickLayout L;
     L.edges = L.zw = L.xw = L.yw = L.edge_groups = 0;
+    L.band = std::min(P.nx, std::min(P.ny, P.nz)) >= 16 ? 4 : 2;
     if (P.nx >= 4 && P.ny >= 4 && P.nz >= 4) {
-        // 16 lines per edge family (4 x 4 band coordinates); lines along x
+        // (2 band)^2 lines per edge family; lines along x
         // and y leave out their band ends, which lie on the lines along z
         // or at a corner
-        L.zw = (P.nz + 63) / 64;
-        L.xw = (P.nx - 4 + 63) / 64;
-        L.yw = (P.ny - 4 + 63) / 64;
-        L.edges = 16 * (L.zw + L.xw + L.yw);
+        L.zw = (P.nz + kEdgeVoxels - 1) / kEdgeVoxels;
+        L.xw = (P.nx - 2 * L.band + kEdgeVoxels - 1) / kEdgeVoxels;
+        L.yw = (P.ny - 2 * L.band + kEdgeVoxels - 1) / kEdgeVoxels;
+        L.edges = 4 * L.band * L.band * (L.zw + L.xw + L.yw);
         L.edge_groups = ((L.edges + 3) / 4 + kXcds - 1) / kXcds * kXcds;
     }
     L.nx = (P.nx + 7) / 8;
@@ -613,43 +642,47 @@ BrickLayout brick_layout(const Params &P) {
     return L;
 }
 
-// Band coordinate q in 0..3 of an axis of n >= 4 samples: 0, 1, n-2, n-1.
-__device__ __forceinline__ int band(int q, int n) { return q < 2 ? q : n - 4 + q; }
+// Band coordinate q in [0, 2 band) of an axis of n samples: the band samples
+// at either face.
+__device__ __forceinline__ int band_coordinate(const BrickLayout &L, int q, int n) {
+    return q < L.band ? q : n - 2 * L.band + q;
+}
 
-__device__ __forceinline__ bool in_band(int i, int n) { return i <= 1 || i >= n - 2; }
+__device__ __forceinline__ bool in_band(const BrickLayout &L, int i, int n) { return i < L.band || i >= n - L.band; }
 
 // A voxel on an edge line: two of its coordinates in the band.
-__device__ __forceinline__ bool on_edge(const int *i, const int *n) {
-    const bool x = in_band(i[0], n[0]), y = in_band(i[1], n[1]), z = in_band(i[2], n[2]);
+__device__ __forceinline__ bool on_edge(const BrickLayout &L, const int *i, const int *n) {
+    const bool x = in_band(L, i[0], n[0]), y = in_band(L, i[1], n[1]), z = in_band(L, i[2], n[2]);
     return (x && y) || (y && z) || (x && z);
 }
 
-// Voxel of lane `lane` of edge wave e; false past the line's end.  Lines
-// along z take every z at band (x, y); lines along x take x in [2, n-3] at
-// band (y, z); lines along y take y in [2, n-3] at band (x, z).
-__device__ __forceinline__ bool edge_voxel(const BrickLayout &L, const int *n, int e, int lane, int *i) {
+// Voxel `slot` (below kEdgeVoxels) of edge wave e; false past the line's end.
+// Lines along z take every z at band (x, y); lines along x take the x outside
+// the bands at band (y, z); lines along y take the y outside at band (x, z).
+__device__ __forceinline__ bool edge_voxel(const BrickLayout &L, const int *n, int e, int slot, int *i) {
     if (e >= L.edges) return false;
-    if (e < 16 * L.zw) {
+    const int side = 2 * L.band, lines = side * side;
+    if (e < lines * L.zw) {
         const int line = e / L.zw, seg = e - line * L.zw;
-        i[0] = band(line & 3, n[0]);
-        i[1] = band(line >> 2, n[1]);
-        i[2] = seg * 64 + lane;
+        i[0] = band_coordinate(L, line % side, n[0]);
+        i[1] = band_coordinate(L, line / side, n[1]);
+        i[2] = seg * kEdgeVoxels + slot;
         return i[2] < n[2];
     }
-    e -= 16 * L.zw;
-    if (e < 16 * L.xw) {
+    e -= lines * L.zw;
+    if (e < lines * L.xw) {
         const int line = e / L.xw, seg = e - line * L.xw;
-        i[1] = band(line & 3, n[1]);
-        i[2] = band(line >> 2, n[2]);
-        i[0] = 2 + seg * 64 + lane;
-        return i[0] < n[0] - 2;
+        i[1] = band_coordinate(L, line % side, n[1]);
+        i[2] = band_coordinate(L, line / side, n[2]);
+        i[0] = L.band + seg * kEdgeVoxels + slot;
+        return i[0] < n[0] - L.band;
     }
-    e -= 16 * L.xw;
+    e -= lines * L.xw;
     const int line = e / L.yw, seg = e - line * L.yw;
-    i[0] = band(line & 3, n[0]);
-    i[2] = band(line >> 2, n[2]);
-    i[1] = 2 + seg * 64 + lane;
-    return i[1] < n[1] - 2;
+    i[0] = band_coordinate(L, line % side, n[0]);
+    i[2] = band_coordinate(L, line / side, n[2]);
+    i[1] = L.band + seg * kEdgeVoxels + slot;
+    return i[1] < n[1] - L.band;
 }
 
 // Brick of workgroup b (counted after the edge section); false for padding
@@ -714,7 +747,7 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Params P, const GatherRa
     Voxel vx;
     // no barriers below: lanes without a voxel return
     if ((int)blockIdx.x < L.edge_groups) {
-        if (!edge_voxel(L, n, 4 * (int)blockIdx.x + w, l, vx.i)) return;
+        if (!edge_voxel(L, n, 4 * (int)blockIdx.x + w, l >> 2, vx.i)) return;
     } else {
         int bx, by, bz;
         if (!brick_of(L, (int)blockIdx.x - L.edge_groups, bx, by, bz)) return;  // uniform per workgroup
@@ -722,28 +755,43 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(Params P, const GatherRa
         vx.i[1] = by * 8 + (w >> 1) * 4 + ((l >> 2) & 3);
         vx.i[2] = bz * 4 + (l >> 4);
         if (vx.i[0] >= n[0] || vx.i[1] >= n[1] || vx.i[2] >= n[2]) return;
-        if (L.edges > 0 && on_edge(vx.i, n)) return;  // gathered by the edge section
+        if (L.edges > 0 && on_edge(L, vx.i, n)) return;  // gathered by the edge section
     }
     for (int a = 0; a < 3; ++a) {
         vx.c[a] = (double)vx.i[a];
         vx.lo[a] = vx.i[a] <= 1 ? -0.5 : (double)(vx.i[a] - 1);
         vx.hi[a] = vx.i[a] >= n[a] - 2 ? (double)n[a] - 0.5 : (double)(vx.i[a] + 1);
     }
+    const bool edge = (int)blockIdx.x < L.edge_groups;
     double total;
     if constexpr (SIMPLE) {
         // axes on which every voxel of the wave is at least two samples
         // from both grid faces (uniform over the wave)
         int mask = 0;
         for (int a = 0; a < 3; ++a) mask |= __all(vx.i[a] >= 2 && vx.i[a] <= n[a] - 3) ? 1 << a : 0;
-        switch (mask) {
-            case 0: total = gather_voxel<kMasked, 0>(P, rays, views, vx); break;
-            case 1: total = gather_voxel<kMasked, 1>(P, rays, views, vx); break;
-            case 2: total = gather_voxel<kMasked, 2>(P, rays, views, vx); break;
-            case 3: total = gather_voxel<kMasked, 3>(P, rays, views, vx); break;
-            case 4: total = gather_voxel<kMasked, 4>(P, rays, views, vx); break;
-            case 5: total = gather_voxel<kMasked, 5>(P, rays, views, vx); break;
-            case 6: total = gather_voxel<kMasked, 6>(P, rays, views, vx); break;
-            default: total = gather_voxel<kMasked, 7>(P, rays, views, vx); break;
+        if (edge) {
+            switch (mask) {
+                case 0: total = gather_voxel<kMasked, 0, true>(P, rays, views, vx); break;
+                case 1: total = gather_voxel<kMasked, 1, true>(P, rays, views, vx); break;
+                case 2: total = gather_voxel<kMasked, 2, true>(P, rays, views, vx); break;
+                case 3: total = gather_voxel<kMasked, 3, true>(P, rays, views, vx); break;
+                case 4: total = gather_voxel<kMasked, 4, true>(P, rays, views, vx); break;
+                case 5: total = gather_voxel<kMasked, 5, true>(P, rays, views, vx); break;
+                case 6: total = gather_voxel<kMasked, 6, true>(P, rays, views, vx); break;
+                default: total = gather_voxel<kMasked, 7, true>(P, rays, views, vx); break;
+            }
+            if (l & 3) return;  // the quad's first lane writes
+        } else {
+            switch (mask) {
+                case 0: total = gather_voxel<kMasked, 0>(P, rays, views, vx); break;
+                case 1: total = gather_voxel<kMasked, 1>(P, rays, views, vx); break;
+                case 2: total = gather_voxel<kMasked, 2>(P, rays, views, vx); break;
+                case 3: total = gather_voxel<kMasked, 3>(P, rays, views, vx); break;
+                case 4: total = gather_voxel<kMasked, 4>(P, rays, views, vx); break;
+                case 5: total = gather_voxel<kMasked, 5>(P, rays, views, vx); break;
+                case 6: total = gather_voxel<kMasked, 6>(P, rays, views, vx); break;
+                default: total = gather_voxel<kMasked, 7>(P, rays, views, vx); break;
+            }
         }
     } else {
         total = gather_voxel<kGeneral>(P, rays, views, vx);
