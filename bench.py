@@ -148,7 +148,7 @@ def record_counters(paths, calibration_bytes: float) -> int:
     kernels = {}
     for path in paths:
         rows = _counter_rows(path)
-        projector = {k: v for k, v in rows.items() if "forward32" in k[1] or "vjp32" in k[1]}
+        projector = {k: v for k, v in rows.items() if any(n in k[1] for n in ("forward32", "vjp32", "vol_walk"))}
         if not projector:
             copy = max(rows.values(), key=lambda c: c.get("FETCH_SIZE", 0.0) + c.get("WRITE_SIZE", 0.0))
             if calibration_bytes > 0 and copy.get("FETCH_SIZE"):
@@ -943,8 +943,8 @@ def fullscan_guards(grid, geometry, values, samples: int) -> dict:
 
 
 def roofline_report(args, fwd_ms: float, vjp_ms: float, effective: int, half: bool) -> dict:
-    """Roofline of the dominant kernel (the joint VJP at the benchmark's
-    shape).  ``achieved`` is its measured HBM traffic per launch (rocprofv3
+    """Roofline of the dominant part (the joint VJP at the benchmark's shape:
+    the volume and the pose launch together).  ``achieved`` is its measured HBM traffic per launch (rocprofv3
     FETCH_SIZE + WRITE_SIZE, calibrated on a copy kernel, recorded in
     profiles/projector_counters.json for the sources digest it was measured
     at) over its launch time (HIP events on its launch stream in the timed
@@ -961,16 +961,20 @@ def roofline_report(args, fwd_ms: float, vjp_ms: float, effective: int, half: bo
 
     gather_b = 16 if half else GATHER_B
     if vjp_ms >= fwd_ms:
-        kernel, ms, per_sample = "vjp32_kernel<float, true, true, 12, false, 2, false>", vjp_ms, gather_b + SCATTER_B
+        parts, ms, per_sample = (["vol_walk_kernel<float, float, false>", "vjp32_kernel<float, 12, false, 3>"], vjp_ms,
+                                 gather_b + SCATTER_B)
     else:
-        kernel, ms, per_sample = "forward32_kernel<float, false, 2, false>", fwd_ms, gather_b
+        parts, ms, per_sample = ["forward32_kernel<float, false, 3>"], fwd_ms, gather_b
+    kernel = " + ".join(parts)
     digest = sources_digest()
     recorded, counters = None, None
     if COUNTERS.exists():
         recorded = json.loads(COUNTERS.read_text())
         if recorded.get("sources_sha256") == digest and not half and args.samples == SAMPLES and \
                 args.views == VIEWS:
-            counters = next((v for k, v in recorded["kernels"].items() if kernel in k), None)
+            found = [next((v for k, v in recorded["kernels"].items() if part in k), None) for part in parts]
+            if all(found):
+                counters = {name: sum(v[name] for v in found) for name in set.intersection(*map(set, found))}
     seconds = ms * 1e-3
     report = {"bound": "hbm", "kernel": kernel, "kernel_ms": round(ms, 3), "forward_kernel_ms": round(fwd_ms, 3),
               "vjp_kernel_ms": round(vjp_ms, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -592,16 +592,17 @@ __device__ __forceinline__ double gather_voxel(const Params &P, const GatherRay 
 // bricks (workgroup b runs on XCD b % 8; surface is padded to a multiple of
 // 8 so that interior workgroups keep that correspondence).
 //
-// The voxels along the grid's 12 edges (two coordinates within two samples
-// of a face) collect the most: every sample of every ray that clips that
-// edge, up to a hundred times an interior voxel.  They go before everything
-// else, each wave taking 16 consecutive voxels along one edge line, a quad of
-// lanes to a voxel: those voxels' pixel windows advance through the same
-// columns (or rows) in step, so their long windows coincide in the wave
-// instead of queueing one after another, and the quad takes four samples a
-// step (24 views of 256^2 at S = 512 into 128^3: with a lane to a voxel the
-// edge waves ran up to 25 ms and the kernel 25.2; 15.5 with quads on the two
-// outermost samples, 8.6 with quads on four, next to which the rest runs 8).  The lanes of surface bricks that fall on an edge line are idle.
+// The voxels along the grid's 12 edges (two coordinates near a face) collect
+// the most: every sample of every ray that clips that edge, up to a hundred
+// times an interior voxel.  They go before everything else, each wave taking 16
+// consecutive voxels along one edge line, a quad of lanes to a voxel: those
+// voxels' pixel windows advance through the same columns (or rows) in step, so
+// their long windows coincide in the wave instead of queueing one after
+// another, and the quad takes four samples a step.  (24 views of 256^2 at S =
+// 512 into 128^3: with a lane to a voxel the edge waves ran up to 25 ms and the
+// kernel 25.2; 15.5 with quads on the two outermost samples, 8.5 on four, 8.2
+// on six, 8.7 on eight.)  The lanes of surface bricks that fall on an edge line
+// are idle.
 constexpr int kEdgeVoxels = 16;  // voxels of an edge wave, a quad of lanes each
 
 struct BrickLayout {
