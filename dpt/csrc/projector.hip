@@ -1767,9 +1767,42 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                     const bool finite = finite_span(o, d, lower, step, 0, P.samples);
                     bad = !finite;
                     const float m = fabsf(volume_factor);
-                    summed = finite && m >= 0x1p-102f && m <= 0x1p96f &&
-                             span_inside(P, o, d, lower, step, 0, P.samples);
+                    summed = finite && m >= 0x1p-102f && m <= 0x1p96f;
                     scattered = !summed;
+                    if (summed && !span_inside(P, o, d, lower, step, 0, P.samples)) {
+                        // rounding put end samples outside (chords of a tenth
+                        // of a voxel and less): the samples inside are a run
+                        const auto inside = [&](int k) {
+                            const float pos = fmaf((float)k + 0.5f, step, lower);
+                            return inside32(P, fmaf(pos, d[0], o[0]), fmaf(pos, d[1], o[1]), fmaf(pos, d[2], o[2]));
+                        };
+                        const int middle = P.samples / 2;
+                        if (inside(middle)) {
+                            int below = 0, above = middle;  // first sample inside
+                            while (below < above) {
+                                const int k = (below + above) >> 1;
+                                if (inside(k))
+                                    above = k;
+                                else
+                                    below = k + 1;
+                            }
+                            walk_first = fmax(walk_first, (double)below);
+                            below = middle;
+                            above = P.samples - 1;  // last sample inside
+                            while (below < above) {
+                                const int k = (below + above + 1) >> 1;
+                                if (inside(k))
+                                    below = k;
+                                else
+                                    above = k - 1;
+                            }
+                            walk_last = fmin(walk_last, (double)(below + 1));
+                            summed = walk_last > walk_first;
+                        } else {
+                            summed = false;
+                            scattered = true;
+                        }
+                    }
                 }
             }
         } else {

@@ -105,3 +105,20 @@ def test_cell_gauss_pieces_match_the_oracle(shape, scale):
     assert not any(status)
     # FP32-rounded increments, then one FP32 rounding of each sum
     assert _rel(actual / scale, expected / scale) <= 1e-7
+
+
+@pytest.mark.parametrize("offset", [2e-2, 2e-3, 1e-4])
+def test_chords_near_the_rounding_of_a_sample(offset):
+    """Rays that clip a vertical edge with chords down to the FP32 rounding of a
+    sample's position: their end samples fall outside the support, the others
+    are one run, added with the rest."""
+    print(f"case walk grazing {offset}", flush=True)
+    grid = O.Grid((6, 20, 20), (1.0, 1.0, 1.0), (-9.5, -9.5, -2.5))
+    z = np.linspace(-2.0, 2.0, 64)
+    corner = 10.0 - offset
+    src = np.stack([np.full(64, corner - 700.0), np.full(64, corner + 700.0), z], 1)
+    end = np.stack([np.full(64, corner + 500.0), np.full(64, corner - 500.0), z], 1)
+    actual, expected = _volume(grid, 1024, "float32", rays=(src, end))
+    # the oracle drops the same end samples; a chord of 2 offset holds the
+    # rounding of its positions, 1e-4 voxel, in weights near one
+    assert _rel(actual, expected) <= 2e-3
