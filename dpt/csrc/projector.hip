@@ -1688,6 +1688,8 @@ __device__ __forceinline__ float walk_fma(float a, float b, float c) { return fm
 __device__ __forceinline__ double walk_fma(double a, double b, double c) { return fma(a, b, c); }
 __device__ __forceinline__ float walk_floor(float a) { return floorf(a); }
 __device__ __forceinline__ double walk_floor(double a) { return floor(a); }
+__device__ __forceinline__ float walk_unit(float a) { return __builtin_amdgcn_fmed3f(a, 0.0f, 1.0f); }
+__device__ __forceinline__ double walk_unit(double a) { return fmin(fmax(a, 0.0), 1.0); }
 
 // Add the brick's non-zero entries to the FP64 accumulator and clear them,
 // 16 lanes to a row of x-adjacent entries: device atomics cost per 64-byte
@@ -1936,24 +1938,30 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
             // as wide as the brick holds
             width = 2 * B.volume <= P.walk_cap ? 2 * (s1 - s0) : s1 - s0;
             s0 = s1;
-            // eight corner sums of a run at mean fractions f, index variance
-            // var and advances b, times g
+            // Mean corner weights of a run at mean fractions f, index variance
+            // var and advances b, times g.  Each is a product of its own
+            // fractions plus the covariances, not a difference of the others,
+            // so a small corner keeps its relative accuracy, and is clamped to
+            // [0, 1] (the mean of weights; an output modifier of the multiply-
+            // add) where the covariances cancel it: sums of a non-negative
+            // image stay non-negative.  Four instructions more than corners
+            // by subtraction.
             auto realised = [&](R x) { return GAUSS ? destination_increment(P, (double)x) : (double)x; };
             auto deposit = [&](const int *l, const R *f, const R *b, R var, R g) {
                 const R fx = f[0], fy = f[1], fz = f[2];
+                const R gx = (R)1 - fx, gy = (R)1 - fy, gz = (R)1 - fz;
                 const R vx = var * b[0], vy = var * b[1];
                 const R exy = vx * b[1], exz = vx * b[2], eyz = vy * b[2];
-                const R mxy = walk_fma(fx, fy, exy), mxz = walk_fma(fx, fz, exz), myz = walk_fma(fy, fz, eyz);
-                const R mxyz = walk_fma(mxy, fz, walk_fma(exz, fy, eyz * fx));
+                const R m[4] = {walk_fma(gx, gy, exy), walk_fma(fx, gy, -exy), walk_fma(gx, fy, -exy),
+                                walk_fma(fx, fy, exy)};
+                const R xf = exz * fy, xg = exz * gy, yf = eyz * fx, yg = eyz * gx;
+                const R u[4] = {-(xg + yg), xg - yf, yg - xf, xf + yf};
                 R c[8];
-                c[7] = mxyz;
-                c[3] = mxy - mxyz;
-                c[5] = mxz - mxyz;
-                c[6] = myz - mxyz;
-                c[1] = (fx - mxy) - c[5];
-                c[2] = (fy - mxy) - c[6];
-                c[4] = (fz - mxz) - c[6];
-                c[0] = (((R)1 - fx) - c[2]) - (c[4] + c[6]);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    c[k] = walk_unit(walk_fma(m[k], gz, -u[k]));
+                    c[k + 4] = walk_unit(walk_fma(m[k], fz, u[k]));
+                }
                 if (use_lds) {
                     const int at = (int)(__umul24(__umul24((unsigned)l[2], (unsigned)B.by) + (unsigned)l[1],
                                                   (unsigned)B.bx) + (unsigned)l[0]) - B.origin;

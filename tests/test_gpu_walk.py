@@ -122,3 +122,72 @@ def test_chords_near_the_rounding_of_a_sample(offset):
     # the oracle drops the same end samples; a chord of 2 offset holds the
     # rounding of its positions, 1e-4 voxel, in weights near one
     assert _rel(actual, expected) <= 2e-3
+
+
+def _corner_rays(exponents, seed):
+    """512 rays of 1/8 mm along x, one in every second cell of a 16^3 unit grid,
+    whose midpoints lie 2^-e short of the cell's far corner on every axis."""
+    rng = np.random.default_rng(seed)
+    k, j, i = (2 * a.ravel() for a in np.meshgrid(*[np.arange(8)] * 3, indexing="ij"))
+    cell = np.stack([i, j, k], 1).astype(np.float64)
+    short = 2.0 ** -rng.integers(*exponents, cell.shape)
+    short[:, 0] += 0.0625  # the whole segment inside the cell
+    middle = cell + 1.0 - short
+    half = np.array([0.0625, 0.0, 0.0])
+    return cell.astype(int), middle - half, middle + half
+
+
+@pytest.mark.parametrize("mode", ["float32", "float64", "cell_gauss"])
+def test_small_corner_sums_keep_sign_and_relative_accuracy(mode):
+    """Corner weights down to the product of three distances 2^-e: the sums of a
+    positive image are positive and accurate to their own size, not to that of
+    the largest corner."""
+    print(f"case walk corners {mode}", flush=True)
+    grid = O.Grid((16, 16, 16), (1.0, 1.0, 1.0))
+    cell, src, end = _corner_rays((4, 12) if mode == "float32" else (4, 24), 1)
+    precision = "float32" if mode == "float32" else "float64"
+    gpu = NativeScene(grid, 1, rays=(src, end), precision=precision,
+                      extra_needs=_native.CELL_GAUSS if mode == "cell_gauss" else 0)
+    actual, _, status = gpu.vjp(np.full(grid.voxels, 0.02, np.float32), np.ones(len(src)), pose_grad=False)
+    assert not any(status)
+    actual = actual.reshape(grid.shape).astype(np.float64)
+    fraction = 0.5 * (src + end) - cell  # exact
+    for corner in range(8):
+        bits = [corner >> a & 1 for a in range(3)]
+        weight = np.prod([fraction[:, a] if bits[a] else 1.0 - fraction[:, a] for a in range(3)], axis=0)
+        at = cell + np.array(bits)
+        got = actual[at[:, 2], at[:, 1], at[:, 0]]
+        assert np.all(got >= 0.0), (corner, got.min())
+        # three products, the factor and the gradient, rounded to 24 bits each
+        np.testing.assert_allclose(got, 0.125 * weight, rtol=6 * 2.0 ** -24, atol=0, err_msg=str(bits))
+
+
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+@pytest.mark.parametrize("samples", [2, 3, 8, 500])
+def test_corner_sums_of_oblique_runs_stay_non_negative(samples, precision):
+    """Runs from near one corner of a cell to near the opposite one, where the
+    covariances cancel the products of the mean fractions."""
+    print(f"case walk oblique runs S={samples} {precision}", flush=True)
+    grid = O.Grid((16, 16, 16), (1.0, 1.0, 1.0))
+    rng = np.random.default_rng(samples)
+    cell = _corner_rays((4, 5), 0)[0].astype(np.float64)
+    near = rng.integers(0, 2, cell.shape)
+    slack = 2.0 ** -rng.integers(3, 13, (2, *cell.shape))
+    src = cell + np.where(near, 1.0 - slack[0], slack[0])
+    end = cell + np.where(near, slack[1], 1.0 - slack[1])
+    gpu = NativeScene(grid, samples, rays=(src, end), precision=precision)
+    actual, _, status = gpu.vjp(np.full(grid.voxels, 0.02, np.float32), np.ones(len(src)), pose_grad=False)
+    assert not any(status)
+    actual = actual.reshape(grid.shape).astype(np.float64)
+    assert actual.min() >= 0.0
+    at = (np.arange(samples) + 0.5)[:, None, None] / samples
+    fraction = src + at * (end - src) - cell
+    length = np.linalg.norm(end - src, axis=1)
+    for corner in range(8):
+        bits = [corner >> a & 1 for a in range(3)]
+        weight = np.prod([fraction[..., a] if bits[a] else 1.0 - fraction[..., a] for a in range(3)], axis=0).mean(0)
+        v = cell.astype(int) + np.array(bits)
+        # FP32 rays: positions up to 16 at 2^-24 in origin and direction; the
+        # covariances leave at least an eighth of the products at these slacks
+        np.testing.assert_allclose(actual[v[:, 2], v[:, 1], v[:, 0]], length * weight, rtol=1e-6,
+                                   atol=6e-7 if precision == "float32" else 1e-15, err_msg=str(bits))
