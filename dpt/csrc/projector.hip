@@ -2009,7 +2009,9 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                         next_t[a] = (plane[a] - W.A[a]) * inv[a];
                     }
                 }
-                // every step passes a plane or ends the slab
+                // every step passes a plane or ends the slab; one that does not
+                // advance (planes closer than the rounding of the ray
+                // parameter) flags the view, as in the other kernels of the rule
                 for (int left = P.nx + P.ny + P.nz + 8; t0 < k1 && left > 0; --left) {
                     const double t1 = fmin(fmin(next_t[0], next_t[1]), fmin(next_t[2], k1));
                     if (t1 > t0) {
@@ -2023,6 +2025,8 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                         }
                         clamp_cell(l, f, b);
                         deposit(l, f, b, radius * radius * (1.0 / 3.0), 2.0 * (radius * volume_factor));
+                    } else {
+                        bad = true;
                     }
 #pragma unroll
                     for (int a = 0; a < 3; ++a)
@@ -2032,6 +2036,7 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                         }
                     t0 = fmax(t0, t1);
                 }
+                bad |= t0 < k1;
             } else {
                 // ---- one step per cell
                 R kf = (R)k0;

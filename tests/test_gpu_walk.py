@@ -191,3 +191,23 @@ def test_corner_sums_of_oblique_runs_stay_non_negative(samples, precision):
         # covariances leave at least an eighth of the products at these slacks
         np.testing.assert_allclose(actual[v[:, 2], v[:, 1], v[:, 0]], length * weight, rtol=1e-6,
                                    atol=6e-7 if precision == "float32" else 1e-15, err_msg=str(bits))
+
+
+@pytest.mark.parametrize("distance", [1e15, 3e16, 4e17])
+def test_cell_gauss_pieces_that_do_not_advance_flag_the_view(distance):
+    """Rays from so far away that neighbouring planes share a ray parameter (one
+    ulp of it is 0.2, 7 and 90 grid samples): the volume adjoint alone reports
+    what the image and the joint adjoint report."""
+    print(f"case walk gauss progress {distance}", flush=True)
+    grid = O.Grid((6, 7, 4000), (1.0, 1.0, 1.0))
+    values = np.full(grid.voxels, 0.02, np.float32)
+    rng = np.random.default_rng(3)
+    for _ in range(12):
+        y0, y1, z = rng.uniform(0.0, 6.0), rng.uniform(0.0, 6.0), rng.uniform(0.0, 5.0)
+        rays = (np.array([[-distance, y0, z]]), np.array([[distance, y1, z]]))
+        _, expected = O.Scene(grid, 7, rays=rays).forward(values, precision="fp64", integration="cell_gauss")
+        assert bool(expected[0]) == (distance > 1e15)
+        gpu = NativeScene(grid, 7, rays=rays, precision="float64", extra_needs=_native.CELL_GAUSS)
+        for pose_grad in (False, True):
+            _, _, status = gpu.vjp(values, np.ones(1), pose_grad=pose_grad)
+            assert status.tolist() == expected.tolist(), (y0, y1, z, pose_grad)
