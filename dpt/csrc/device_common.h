@@ -42,7 +42,7 @@ struct Params {
     int vb;                  // views per workgroup (1, 2 or 4): one wave64 per view when > 1
     int tile_w, tile_h;      // pixels per workgroup tile of one view
     int tiles_x, tiles_y, tiles_per_group, total_tiles, chunk;
-    int by_rows;             // 1: XCDs take rows of tiles in turn, not contiguous runs of the walk
+    int row_pitch;           // rows of tiles per view dealt to the XCDs in turn, blank ones included (0: contiguous runs)
     int segments;            // volume adjoint: workgroups per tile, each over its own range of samples
     int base_tiles;          // tiles of one segment (total_tiles / segments)
     int segment_samples;     // samples per segment (a multiple of chunk_samples)
@@ -119,18 +119,19 @@ __device__ __forceinline__ bool finite3d(const double *v) {
 // pose partials.  Explicit ray bundles use 256 consecutive rays per workgroup.
 // Returns false when the whole workgroup lies past the end of the walk.
 //
-// Launches of few views hand out single rows of tiles instead (P.by_rows):
-// rays that meet the volume crowd the middle of a panel, so contiguous runs
-// left most XCDs idle.  One 512^2 view of a
-// 512 x 512 x 139 grid, whole call: 2.76 -> 1.98 ms; 24 views and more keep the
-// runs, whose L2s hold a part of the volume each (FP64 24 x 256^2 over 128^3:
-// 4.7 ms, by rows 5.8).
-__device__ __forceinline__ int walk_index(int b, int chunk, int row, bool by_rows) {
-    const int xcd = b % kXcds, i = b / kXcds;
-    return by_rows ? ((i / row) * kXcds + xcd) * row + i % row : xcd * chunk + i;
-}
+// Launches of few views deal single rows of tiles to the XCDs in turn instead
+// (P.row_pitch): rays that meet the volume crowd the middle of a panel, so
+// contiguous runs leave most XCDs idle.  A view's rows are followed by blank
+// ones up to row_pitch, so that the middle rows of consecutive views fall on
+// different XCDs: without them, panels of 8k rows of tiles put those of every
+// view on the same few (5 views of 256^2 over 139 x 512 x 512 at S = 1024, a
+// lane per ray: contiguous 0.78 ms, rows without blanks 2.79, with them 0.76).
 __device__ __forceinline__ int tile_index(const Params &P) {
-    return walk_index(blockIdx.x, P.chunk, P.tiles_x, P.by_rows);
+    const int xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds;
+    if (P.row_pitch == 0) return xcd * P.chunk + i;
+    const int turn = i / P.tiles_x, dealt = turn * kXcds + xcd;
+    const int group = dealt / P.row_pitch, row = dealt - group * P.row_pitch;
+    return row < P.tiles_y ? (group * P.tiles_y + row) * P.tiles_x + (i - turn * P.tiles_x) : INT_MAX;
 }
 __device__ __forceinline__ bool lane_ray(const Params &P, int &view, int &row, int &col, int &wslot,
                                          bool &wave_valid) {

@@ -2403,14 +2403,29 @@ unsigned grid_blocks(int64_t n) {
     return (unsigned)b;
 }
 
-// XCD walk of a launch (walk_index): rows of tiles in turn for few views with
-// rows for every XCD, else contiguous runs.
-constexpr int kFewViews = 2 * kXcds;
-bool rows_in_turn(int views, int rows) { return views < kFewViews && rows >= 2 * kXcds; }
-void set_walk(Params &P) {
+// XCD walk of a launch (tile_index): rows of tiles in turn for few views with
+// rows for every XCD, else contiguous runs.  A workgroup per wave tile
+// (`wave_tiles`, the split kernels) gains up to 15 views, a lane per ray only
+// below the eight whose runs give every XCD about a view of its own.  MI355X,
+// rows against runs, geometric mean (worst) over 128^3, 139 x 512 x 512 and 97
+// x 181 x 203 and panels of 128^2 to 512^2: split forward at 1 / 3 / 5 / 8 /
+// 15 views 0.72 (1.00) / 0.63 (0.89) / 0.82 (1.00) / 0.97 (1.01) / 0.92
+// (0.95), lane-per-ray forward at 3 / 4 / 5 / 7 / 8 views 0.52 (0.70) / 1.01
+// (1.09) / 0.73 (0.87) / 0.92 (1.25) / 1.02 (1.72), volume walk at 1 / 3 / 5 /
+// 8 views 0.96 (1.08) / 0.94 (1.06) / 0.97 (1.06) / 0.99 (1.05).
+// Row pitch 5 (mod 8) spreads a few views over the XCDs; at seven views of a
+// lane per ray an odd pitch, most often no blank row, keeps an XCD on
+// neighbouring rows of consecutive views (7 views of 257 x 301 over 97 x 181 x
+// 203: pose adjoint 0.43 ms, with pitch 5 0.62).
+void set_walk(Params &P, bool wave_tiles = false) {
     const int rows = P.total_tiles / P.tiles_x;
-    P.by_rows = rows_in_turn(P.views, rows);
-    P.chunk = P.by_rows ? (rows + kXcds - 1) / kXcds * P.tiles_x : (P.total_tiles + kXcds - 1) / kXcds;
+    P.row_pitch = 0;
+    P.chunk = (P.total_tiles + kXcds - 1) / kXcds;
+    if (P.bundle || rows < 2 * kXcds || P.views >= (wave_tiles ? 2 * kXcds : kXcds)) return;
+    const bool spread = wave_tiles || P.views < kXcds - 1;
+    P.row_pitch = P.tiles_y;
+    while (spread ? P.row_pitch % kXcds != 5 : P.row_pitch % 2 == 0) ++P.row_pitch;
+    P.chunk = (rows / P.tiles_y * P.row_pitch + kXcds - 1) / kXcds * P.tiles_x;
 }
 
 // Tile geometry for `vb` views per workgroup (see lane_ray).
@@ -2582,8 +2597,9 @@ unsigned tile_grid(const Params &P) { return (unsigned)(P.chunk * kXcds); }
 // One workgroup per wave tile (split_tile).
 Params split_params(Params P) {
     P.tiles_x = P.wt_x;
+    P.tiles_y = P.wt_y;
     P.total_tiles = P.views * P.wt_per_view;
-    set_walk(P);
+    set_walk(P, true);
     return P;
 }
 
