@@ -43,6 +43,7 @@ struct Params {
     int tile_w, tile_h;      // pixels per workgroup tile of one view
     int tiles_x, tiles_y, tiles_per_group, total_tiles, chunk;
     int row_pitch;           // rows of tiles per view dealt to the XCDs in turn, blank ones included (0: contiguous runs)
+    int fp64;                // 1: FP64 sampling
     int segments;            // volume adjoint: workgroups per tile, each over its own range of samples
     int base_tiles;          // tiles of one segment (total_tiles / segments)
     int segment_samples;     // samples per segment (a multiple of chunk_samples)

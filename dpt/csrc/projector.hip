@@ -2404,16 +2404,20 @@ unsigned grid_blocks(int64_t n) {
 }
 
 // XCD walk of a launch (tile_index): rows of tiles in turn for few views with
-// rows for every XCD, else contiguous runs.  A workgroup per wave tile
-// (`wave_tiles`, the split kernels) gains up to 15 views, a lane per ray only
-// below the eight whose runs give every XCD about a view of its own.  MI355X,
-// rows against runs, geometric mean (worst) over 128^3, 139 x 512 x 512 and 97
-// x 181 x 203 and panels of 128^2 to 512^2: split forward at 1 / 3 / 5 / 8 /
-// 15 views 0.72 (1.00) / 0.63 (0.89) / 0.82 (1.00) / 0.97 (1.01) / 0.92
-// (0.95), lane-per-ray forward at 3 / 4 / 5 / 7 / 8 views 0.52 (0.70) / 1.01
-// (1.09) / 0.73 (0.87) / 0.92 (1.25) / 1.02 (1.72), volume walk at 1 / 3 / 5 /
-// 8 views 0.96 (1.08) / 0.94 (1.06) / 0.97 (1.06) / 0.99 (1.05).
-// Row pitch 5 (mod 8) spreads a few views over the XCDs; at seven views of a
+// rows for every XCD, else contiguous runs.  MI355X, rows against runs,
+// geometric mean (worst) over 128^3, 139 x 512 x 512, 97 x 181 x 203 (FP64:
+// 300^3) and panels of 128^2 to 512^2, at 1 / 3 / 5 / 7 / 10 / 15 views: split
+// forward 0.72 (1.00) / 0.63 (0.89) / 0.82 (1.00) / 0.94 (1.10) / 0.87 (0.95) /
+// 0.92 (0.95); FP32 forward of a lane per ray from 3 views 0.52 (0.70) / 0.73
+// (0.87) / 0.92 (1.25) / 0.87 (1.14) / 0.94 (1.15), volume walk 0.96 (1.08) /
+// 0.94 (1.06) / 0.97 (1.06) / 0.99 (1.07) / 0.95 (1.18) / 1.00 (1.10); FP64
+// forward 1.00 (1.20) / 0.78 (1.00) / 0.78 (1.07) / 0.92 (1.26) / 0.87 (1.02) /
+// 0.94 (1.08), exact pose adjoint 0.92 / 0.78 / 0.80 / 0.90 / 0.90 / 1.02 (1.31).
+// Eight FP32 views keep runs, one view to an XCD: on average as fast (0.99),
+// and 8 views of 257 x 301 over 139 x 512 x 512 take 0.89 ms, by rows 1.32.
+// From 24 views on each run's L2 holds a part of the volume (FP64 24 x 256^2
+// over 128^3: 4.7 ms, by rows 5.8).
+// Row pitch 5 (mod 8) spreads a few views over the XCDs; for more views of a
 // lane per ray an odd pitch, most often no blank row, keeps an XCD on
 // neighbouring rows of consecutive views (7 views of 257 x 301 over 97 x 181 x
 // 203: pose adjoint 0.43 ms, with pitch 5 0.62).
@@ -2421,7 +2425,8 @@ void set_walk(Params &P, bool wave_tiles = false) {
     const int rows = P.total_tiles / P.tiles_x;
     P.row_pitch = 0;
     P.chunk = (P.total_tiles + kXcds - 1) / kXcds;
-    if (P.bundle || rows < 2 * kXcds || P.views >= (wave_tiles ? 2 * kXcds : kXcds)) return;
+    if (P.bundle || rows < 2 * kXcds || P.views >= 2 * kXcds) return;
+    if (P.views == kXcds && !P.fp64 && !wave_tiles) return;
     const bool spread = wave_tiles || P.views < kXcds - 1;
     P.row_pitch = P.tiles_y;
     while (spread ? P.row_pitch % kXcds != 5 : P.row_pitch % 2 == 0) ++P.row_pitch;
@@ -2883,6 +2888,7 @@ int plan_create(const dpt_grid_desc *grid, int32_t views, int32_t rows, int32_t 
     P.cols = cols;
     P.samples = samples;
     P.bundle = panels == nullptr ? 1 : 0;
+    P.fp64 = arithmetic == DPT_ARITH_FP64;
     configure_tiles(P, 1);
     P.chunk_samples = chunk_samples(samples, grid->nx, grid->ny, grid->nz);
     if (const char *chunk = std::getenv("DPT_AMD_CHUNK")) {
