@@ -2356,6 +2356,7 @@ struct dpt_plan {
     void *d_copy = nullptr;   // the gather copy
     int vjp_vb = 1;          // views per workgroup of the VJP launches
     int forward_vb = 1;      // views per workgroup of the forward launch
+    double view_gap = 0.0;   // voxels between neighbouring views of a workgroup at the grid's rim
     bool timing = false;
     double *ray_out = nullptr;             // destination of a ray-coordinate VJP (caller's buffer)
     GatherRay *d_gather_rays = nullptr;    // adjoint gather workspace, allocated at its first call
@@ -2458,16 +2459,35 @@ void configure_tiles(Params &P, int vb) {
     P.segment_samples = P.samples;
 }
 
+// Whether the FP32 forward or pose launch runs as a workgroup per wave tile
+// (split kernels).  Never above 8192 waves of a lane per ray (8 per SIMD), always
+// up to 512.  Between, its eightfold ray set-up and its adding wave have to be
+// won back: enough samples a ray, few waves for them (6 a sample) or rays so
+// far apart that every lane misses its own cells (`dense` rays per face of a
+// voxel; denser lanes share the L1's lines and issue bounds the march, the pose
+// march first), and no four views in a workgroup within two voxels of each
+// other, whose waves share cells a workgroup per wave tile fetches again.  MI355X, a lane per ray against
+// split: one 512^2 view over 128^3 at S = 1: forward 14 and 36 us, pose adjoint
+// 33 and 81; S = 256: 137 and 103, 157 and 177; over 139 x 512 x 512, S = 64:
+// 109 and 79, 124 and 108; 2000 views of 16^2 over 32^3, S = 128: 131 and 179,
+// 181 and 329.  Over 1458 such points (1 to 2000 views, S 1 to 1024, 32^3 to
+// 256^3) the rule is 2 % off the better of both, split wherever it fits 9 %
+// (forward) and 19 % (pose), a lane per ray 34 % and 31 %.
+bool split_launch(const dpt_plan *p, const Params &P, bool pose) {
+    const long long waves = (long long)P.total_tiles * (kBlock / 64);
+    if (waves > 8192) return false;
+    if (waves <= 512) return true;
+    if (P.samples < (pose ? 48 : 32) || (P.vb == 4 && p->view_gap < 2.0)) return false;
+    const double side = std::cbrt((double)P.nx * P.ny * P.nz);
+    const double rays_per_face = (double)P.vb * P.rows * P.cols / (side * side), dense = pose ? 4.5 : 32.0;
+    return waves <= 6LL * P.samples || rays_per_face <= dense;
+}
+
 // Sample-range segments of the volume adjoint: a launch of few tiles (one view
 // of 512^2 is 1024 workgroups, one wave per SIMD) runs each tile as `segments`
 // workgroups over consecutive ranges of whole chunks (at least two chunks and
 // 256 samples each), aiming at 16384 waves.  DPT_AMD_VJP_SEGMENTS overrides
 // the count (1..8; not the two-chunk floor).
-// A launch of at most 8192 waves (8 per SIMD): one whose sample loops expose
-// their memory latency.
-// (7 views of 257 x 301, 9064 waves, run 7 % slower split.)
-bool small_launch(const Params &P) { return (long long)P.total_tiles * (kBlock / 64) <= 8192; }
-
 void configure_segments(Params &P) {
     const long long waves = (long long)P.total_tiles * (kBlock / 64);
     int g = 1;
@@ -2489,13 +2509,11 @@ void configure_segments(Params &P) {
     set_walk(P);
 }
 
-// Views share a workgroup (and its LDS brick) only when their central rays
-// differ by at most ~4 degrees: then their samples of one chunk overlap.
-int choose_views_per_block(const double *panels, int views, int rows, int cols) {
-    if (views < 2) return 1;
+// Least cosine between the central rays of two views of one group of `vb`
+// consecutive views.
+double least_cosine(const double *panels, int views, int rows, int cols, int vb) {
     std::vector<double> dir(3 * (size_t)views);
-    const int n = views;
-    for (int v = 0; v < n; ++v) {
+    for (int v = 0; v < views; ++v) {
         const double *pn = panels + 12 * (size_t)v;
         double len = 0.0;
         for (int i = 0; i < 3; ++i) {
@@ -2506,20 +2524,22 @@ int choose_views_per_block(const double *panels, int views, int rows, int cols) 
         len = std::sqrt(len);
         for (int i = 0; i < 3; ++i) dir[3 * v + i] /= len;
     }
+    double least = 1.0;
+    for (int g = 0; g + 1 < views; g += vb)
+        for (int a = g; a < g + vb && a < views; ++a)
+            for (int b = a + 1; b < g + vb && b < views; ++b)
+                least = std::fmin(least, dir[3 * a] * dir[3 * b] + dir[3 * a + 1] * dir[3 * b + 1] +
+                                             dir[3 * a + 2] * dir[3 * b + 2]);
+    return least;
+}
+
+// Views share a workgroup (and its LDS brick) only when their central rays
+// differ by at most ~4 degrees: then their samples of one chunk overlap.
+int choose_views_per_block(const double *panels, int views, int rows, int cols) {
+    if (views < 2) return 1;
     const double cos_limit = std::cos(4.0 * 3.14159265358979323846 / 180.0);
-    for (int vb : {4, 2}) {
-        bool ok = true;
-        for (int g = 0; g + 1 < n && ok; g += vb)
-            for (int a = g; a < g + vb && a < n && ok; ++a)
-                for (int b = a + 1; b < g + vb && b < n; ++b) {
-                    const double c = dir[3 * a] * dir[3 * b] + dir[3 * a + 1] * dir[3 * b + 1] + dir[3 * a + 2] * dir[3 * b + 2];
-                    if (c < cos_limit) {
-                        ok = false;
-                        break;
-                    }
-                }
-        if (ok) return vb;
-    }
+    for (int vb : {4, 2})
+        if (least_cosine(panels, views, rows, cols, vb) >= cos_limit) return vb;
     return 1;
 }
 
@@ -2623,7 +2643,7 @@ int launch_forward(dpt_plan *p, const Params &P, const void *field, void *out, b
     if (p->arithmetic == DPT_ARITH_FP32) {
         float *o = static_cast<float *>(out);
         constexpr bool HALF = !std::is_same<T, float>::value;
-        if (small_launch(P)) {
+        if (split_launch(p, P, false)) {
             const Params Q = split_params(P);
             const dim3 tiles(tile_grid(Q)), lanes(64 * kSplitWaves);
             if (cells)
@@ -2663,7 +2683,7 @@ template <typename T, int C, int LAYOUT>
 void launch_vjp32(dpt_plan *p, const Params &P, const T *f, const float *sd, hipStream_t s) {
     constexpr bool HALF = !std::is_same<T, float>::value;
     double *partials = pose_destination<C>(p);
-    if (small_launch(P)) {
+    if (split_launch(p, P, true)) {
         const Params Q = split_params(P);
         hipLaunchKernelGGL((vjp32_split_kernel<T, C, HALF, LAYOUT>), dim3(tile_grid(Q)), dim3(64 * kSplitWaves), 0, s,
                            Q, f, sd, partials);
@@ -2917,6 +2937,11 @@ int plan_create(const dpt_grid_desc *grid, int32_t views, int32_t rows, int32_t 
         if (!P.bundle && (forced == 1 || forced == 2 || forced == 4)) p->vjp_vb = forced;
     }
     p->forward_vb = p->vjp_vb;
+    if (!P.bundle && views > 1) {
+        const double n[3] = {(double)grid->nx, (double)grid->ny, (double)grid->nz};
+        const double angle = std::acos(std::fmin(1.0, least_cosine(panels, views, rows, cols, 2)));
+        p->view_gap = 0.5 * angle * std::sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    }
     if (const char *vb = std::getenv("DPT_AMD_FORWARD_VIEWS_PER_BLOCK")) {
         const int forced = std::atoi(vb);
         if (!P.bundle && (forced == 1 || forced == 2 || forced == 4)) p->forward_vb = forced;

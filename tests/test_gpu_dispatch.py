@@ -96,3 +96,24 @@ def test_fewer_views_take_no_longer():
         times = [_milliseconds(lambda: call(t)) for t in (few, more)]
         print(f"10 and 16 views: {times}", flush=True)
         assert times[0] <= 1.8 * times[1]
+
+
+def test_few_samples_take_no_longer_than_more_rays():
+    """One sample a ray: two 512^2 views with eight waves to set up each ray took
+    58 us for the image and 134 us for the pose adjoint, where three views with
+    one took 20 and 46."""
+    few, more = (Timed((32, 32, 32), views, 512, 512, 1) for views in (2, 3))
+    for call in (Timed.forward, lambda t: t.vjp(_native.POSE)):
+        times = [_milliseconds(lambda: call(t), 15) for t in (few, more)]
+        print(f"2 and 3 views, one sample: {times}", flush=True)
+        assert times[0] <= 1.4 * times[1]
+
+
+def test_views_that_share_cells_keep_a_workgroup():
+    """2000 views of 16^2 a fifth of a degree apart: the four views of a workgroup
+    share cells; a workgroup per wave tile took 0.33 ms of the pose adjoint, twice
+    2080 views (above the split kernels' range)."""
+    few, more = (Timed((32, 32, 32), views, 16, 16, 128) for views in (2000, 2080))
+    times = [_milliseconds(lambda: t.vjp(_native.POSE), 15) for t in (few, more)]
+    print(f"2000 and 2080 views: {times}", flush=True)
+    assert times[0] <= 1.4 * times[1]
