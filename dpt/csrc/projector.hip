@@ -358,11 +358,11 @@ int choose_brick_cap(const Params &P, const double *panels, int *slab_chunks) {
 }
 
 // Bound one chunk's cells over the workgroup and, when the box fits the LDS
-// brick, describe it.  lo / nhi: this lane's lower cell corner minimum and
+// brick, describe it; e: the box's extents in grid samples.  lo / nhi: this lane's lower cell corner minimum and
 // negated maximum over its chunk samples (INT_MAX when it has none).  Every
 // lane gets the same answer (kept in SGPRs); one barrier.
 __device__ __forceinline__ bool chunk_brick(const Params &P, int (*red)[6], int *lo, int *nhi, int cap, bool unit_x,
-                                            Brick &B, bool *overflow = nullptr, bool pad = false) {
+                                            Brick &B, bool pad, int *e) {
     const int wv = threadIdx.x >> 6;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -383,14 +383,12 @@ __device__ __forceinline__ bool chunk_brick(const Params &P, int (*red)[6], int 
         l[a] = min(min(red[0][a], red[1][a]), min(red[2][a], red[3][a]));
         h[a] = -min(min(red[0][3 + a], red[1][3 + a]), min(red[2][3 + a], red[3][3 + a]));
     }
+    e[0] = e[1] = e[2] = 0;
     if (l[0] == INT_MAX) return false;
     const int n[3] = {P.nx, P.ny, P.nz};
-    int e[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) e[a] = min(h[a] + 1, n[a] - 1) - l[a] + 1;
-    const long long vol = (long long)e[0] * e[1] * e[2];
-    if (overflow != nullptr) *overflow = vol > cap;
-    if (vol > cap) return false;
+    if ((long long)e[0] * e[1] * e[2] > cap) return false;
     // every lane holds the same values: keep them in SGPRs
     B.x0 = __builtin_amdgcn_readfirstlane(l[0]);
     B.y0 = __builtin_amdgcn_readfirstlane(l[1]);
@@ -1639,6 +1637,20 @@ __global__ __launch_bounds__(kBlock, 3) void vjp_gauss_kernel(Params P, const T 
 // costs no lockstep waste; a slab whose box overflows the brick is halved, and
 // the next one doubled while it fits.
 //
+// Where rays lie more than about three voxels apart (kWalkSparse) a brick holds
+// mostly zeros: its box fills the LDS with a slab of a few samples, and the
+// bounds, barriers and drain of every slab cost more than the few sums they
+// merge.  Such a workgroup adds its corner sums by device atomics at once, two
+// x-adjacent entries a request from a pair of lanes; it is found when a slab of
+// eight samples overflows (asked at sixteen, 30 views of 128^2 over 128^3 ran 6
+// % slower; asked at four, 24 views of 128^2 over 256^3 at S = 64 took 4.3
+// instead of 2.1 ms).  MI355X, bricks and atomics: 24 views over 256^3 at S =
+// 512, panels of 96^2 / 128^2 / 160^2 (0.06 / 0.11 / 0.17 rays a voxel) 8.6 and
+// 4.3 / 9.2 and 7.5 / 12.4 and 11.6 ms, of 192^2 (0.25) 8.5 and 16.4; 60 views
+// of 24^2 over 128^3 3.9 and 0.45 ms; 24 x 256^2 over 512^3 at S = 128 33.7 and
+// 12.6; 2^18 random rays in 256^3 5.8 and 2.2; 2^16 by the exact rule in 128^3
+// 1.51 and 0.49.
+//
 // Bound by the device atomics of the drain (one request per 64-byte block,
 // 23.6 G/s), the LDS atomics and VALU issue, in turn.  MI355X, before (per
 // sample, joint with the pose) and after (walk + pose launch): 360-view 512^2
@@ -1654,6 +1666,7 @@ constexpr double kWalkBias = 0x1.8p20;         // 1.5 * 2^20: a sum's low word i
 constexpr int kWalkBiasHigh = 0x41380000;      // high word of the bias: the difference is floor(coordinate)
 constexpr int kWalkWidth = 16;                  // grid samples of the first slab
 constexpr int kWalkMaxAxis = 1 << 18;          // largest axis of the biased form
+constexpr float kWalkSparse = 0.12f;           // least rays per grid sample of a slab's cross-section worth a brick
 
 // Floor and fraction of coordinate a of sample k (R float: through the bias,
 // 2^-32 resolution; R double: exact).
@@ -1691,6 +1704,14 @@ __device__ __forceinline__ double walk_floor(double a) { return floor(a); }
 __device__ __forceinline__ float walk_unit(float a) { return __builtin_amdgcn_fmed3f(a, 0.0f, 1.0f); }
 __device__ __forceinline__ double walk_unit(double a) { return fmin(fmax(a, 0.0), 1.0); }
 
+// The value of the other lane of a pair of lanes (quad_perm [1, 0, 3, 2]); both
+// must be active.
+__device__ __forceinline__ int pair_lane(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true); }
+__device__ __forceinline__ float pair_lane(float v) { return __int_as_float(pair_lane(__float_as_int(v))); }
+__device__ __forceinline__ double pair_lane(double v) {
+    return __hiloint2double(pair_lane(__double2hiint(v)), pair_lane(__double2loint(v)));
+}
+
 // Add the brick's non-zero entries to the FP64 accumulator and clear them,
 // 16 lanes to a row of x-adjacent entries: device atomics cost per 64-byte
 // block (23.6 G blocks/s measured, whether 1 or 8 entries of it are added).
@@ -1721,11 +1742,15 @@ __device__ __forceinline__ void walk_drain(const Params &P, const Brick &B, doub
 // are a run of two samples with index variance radius^2 / 3 (24 views of 256^2
 // over 128^3: joint adjoint 4.15 -> 1.74 + 1.05 ms; two products a corner and
 // node and 6.1e7 device atomics before).
+// FP32 sums keep six waves per SIMD (80 VGPRs, 32 bytes of spills; 90 and five
+// without the bound: full scan 61.9 and 62.9 ms), FP64 ones take four (121; five
+// spill 92 bytes: 24 views of 256^2 over 128^3 by the exact rule 1.25 and 1.40
+// ms).
 template <typename S, typename R, bool GAUSS = false>
-__global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__restrict__ seeds,
+__global__ __launch_bounds__(kBlock, (std::is_same<R, float>::value ? 6 : 4)) void vol_walk_kernel(Params P, const S *__restrict__ seeds,
                                                           double *__restrict__ acc) {
     extern __shared__ double brick[];
-    __shared__ int bound_red[kBlock / 64][6];
+    __shared__ int bound_red[kBlock / 64][6], ray_red[kBlock / 64];
     int view, row, col, wslot;
     bool wave_valid;
     if (!lane_ray(P, view, row, col, wslot, wave_valid)) return;
@@ -1903,40 +1928,73 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
         }
         const int cap[3] = {P.capx, P.capy, P.capz};
         int width = GAUSS ? max(1, (slab_hi - slab_lo) / P.gauss_chunks) : kWalkWidth;
+        // where the walk crosses slab coordinate b; `whole`: the first sample beyond it
+        auto crossing = [&](int b, bool whole) {
+            double t = ((double)b - slab_A) * slab_inv;
+            if (whole) t = up ? ceil(t) : floor(t) + 1.0;
+            return fmin(fmax(t, walk_first), walk_last);
+        };
+        auto cell_bounds = [&](double k0, double k1, bool inclusive, int *blo, int *bnhi) {
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                blo[a] = bnhi[a] = INT_MAX;
+                if (k1 > k0) {
+                    const int la = walk_lower<R>(W.A[a], W.B[a], k0, cap[a]);
+                    const int lb = walk_lower<R>(W.A[a], W.B[a], inclusive ? k1 : k1 - 1.0, cap[a]);
+                    blo[a] = min(la, lb);
+                    bnhi[a] = -max(la, lb);
+                }
+            }
+        };
+        // the rays through a thin slab in the middle against the cross-section
+        // of its box (one barrier before, one after the bound's own)
+        auto too_sparse = [&]() {
+            const int m0 = (slab_lo + slab_hi) / 2 - 2;
+            const double t0 = crossing(m0, false), t1 = crossing(m0 + 4, false);
+            const double k0 = fmin(t0, t1), k1 = summed ? fmax(t0, t1) : k0;
+            const int rays = __popcll(__builtin_amdgcn_ballot_w64(k1 > k0));
+            int blo[3], bnhi[3], e[3];
+            cell_bounds(k0, k1, true, blo, bnhi);
+            __syncthreads();  // the bound rewrites bound_red
+            if (lane == 0) ray_red[wv] = rays;
+            Brick B{};
+            (void)chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, true, e);
+            const float across = axis == 0 ? (float)e[1] * e[2] : (axis == 1 ? (float)e[0] * e[2] : (float)e[0] * e[1]);
+            const bool sparse = (float)(ray_red[0] + ray_red[1] + ray_red[2] + ray_red[3]) < kWalkSparse * across;
+            return (bool)__builtin_amdgcn_readfirstlane(sparse);
+        };
+        bool weighed = false, sparse = false;  // asked once, when a thin slab's box overflows the brick
         for (int s0 = slab_lo; s0 < slab_hi;) {
             // ---- this slab's samples [k0, k1) of the lane and its brick
-            double k0 = 0.0, k1 = 0.0, next;
+            double k0, k1, next;
             int s1;
+            long long box;
             Brick B{};
             bool use_lds;
             for (;;) {
-                s1 = min(s0 + width, slab_hi);
-                double t = ((double)s1 - slab_A) * slab_inv;
-                if constexpr (!GAUSS) t = up ? ceil(t) : floor(t) + 1.0;
-                t = fmin(fmax(t, walk_first), walk_last);
-                if (s1 == slab_hi) t = up ? walk_last : walk_first;
+                s1 = sparse ? slab_hi : min(s0 + width, slab_hi);  // sparse: all that is left
+                const double t = s1 == slab_hi ? (up ? walk_last : walk_first) : crossing(s1, !GAUSS);
                 next = up ? fmax(t, done) : fmin(t, done);
                 k0 = fmin(next, done);
                 k1 = summed ? fmax(next, done) : k0;
-                int blo[3] = {INT_MAX, INT_MAX, INT_MAX}, bnhi[3] = {INT_MAX, INT_MAX, INT_MAX};
-                if (k1 > k0) {
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        const int la = walk_lower<R>(W.A[a], W.B[a], k0, cap[a]);
-                        const int lb = walk_lower<R>(W.A[a], W.B[a], GAUSS ? k1 : k1 - 1.0, cap[a]);
-                        blo[a] = min(la, lb);
-                        bnhi[a] = -max(la, lb);
-                    }
-                }
-                bool overflow = false;
-                use_lds = chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, &overflow, true);
-                if (!overflow || s1 - s0 <= 1) break;
+                use_lds = false;
+                box = 0;
+                if (sparse) break;
+                int blo[3], bnhi[3], e[3];
+                cell_bounds(k0, k1, GAUSS, blo, bnhi);
+                use_lds = chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, true, e);
+                box = (long long)e[0] * e[1] * e[2];
+                if (box <= P.walk_cap || s1 - s0 <= 1) break;
                 width = max(1, (s1 - s0) >> 1);
+                if (!weighed && s1 - s0 <= kWalkWidth / 2) {
+                    weighed = true;
+                    sparse = too_sparse();
+                }
                 __syncthreads();  // the next bound rewrites bound_red
             }
             done = next;
             // as wide as the brick holds
-            width = 2 * B.volume <= P.walk_cap ? 2 * (s1 - s0) : s1 - s0;
+            width = 2 * (use_lds ? (long long)B.volume : box) <= P.walk_cap ? 2 * (s1 - s0) : s1 - s0;
             s0 = s1;
             // Mean corner weights of a run at mean fractions f, index variance
             // var and advances b, times g.  Each is a product of its own
@@ -1947,7 +2005,11 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
             // image stay non-negative.  Four instructions more than corners
             // by subtraction.
             auto realised = [&](R x) { return GAUSS ? destination_increment(P, (double)x) : (double)x; };
-            auto deposit = [&](const int *l, const R *f, const R *b, R var, R g) {
+            // IN_BRICK: into the brick.  Otherwise by device atomics, and the
+            // whole wave calls: the two lanes of a pair add the x-adjacent
+            // entries of the even lane's rows, then of the odd lane's, one
+            // request for both entries (a lane without a run adds nothing).
+            auto deposit = [&](auto in_brick, bool live, const int *l, const R *f, const R *b, R var, R g) {
                 const R fx = f[0], fy = f[1], fz = f[2];
                 const R gx = (R)1 - fx, gy = (R)1 - fy, gz = (R)1 - fz;
                 const R vx = var * b[0], vy = var * b[1];
@@ -1962,7 +2024,7 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                     c[k] = walk_unit(walk_fma(m[k], gz, -u[k]));
                     c[k + 4] = walk_unit(walk_fma(m[k], fz, u[k]));
                 }
-                if (use_lds) {
+                if constexpr (decltype(in_brick)::value) {
                     const int at = (int)(__umul24(__umul24((unsigned)l[2], (unsigned)B.by) + (unsigned)l[1],
                                                   (unsigned)B.bx) + (unsigned)l[0]) - B.origin;
 #pragma unroll
@@ -1970,11 +2032,17 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                         atomicAdd(&brick[at + ((k & 1) ? B.lsx : 0) + ((k & 2) ? B.lsy : 0) + ((k & 4) ? B.lsz : 0)],
                                   realised(g * c[k]));
                 } else {
-                    const int at = (l[2] * P.ny + l[1]) * P.nx + l[0];
+                    const bool odd = lane & 1;
+                    const int at = (l[2] * P.ny + l[1]) * P.nx + l[0], pair = pair_lane(at);
+                    const int even_at = odd ? pair + P.sx : at, odd_at = odd ? at + P.sx : pair;
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        const double v = realised(g * c[k]);
-                        if (v != 0.0) unsafeAtomicAdd(&acc[at + corner_offset(P, k)], v);
+                    for (int k = 0; k < 8; k += 2) {
+                        const R low = live ? g * c[k] : (R)0, high = live ? g * c[k + 1] : (R)0;
+                        const R from = pair_lane(odd ? low : high);
+                        const double even_sum = realised(odd ? from : low), odd_sum = realised(odd ? high : from);
+                        const int row = corner_offset(P, k);
+                        if (even_sum != 0.0) unsafeAtomicAdd(&acc[even_at + row], even_sum);
+                        if (odd_sum != 0.0) unsafeAtomicAdd(&acc[odd_at + row], odd_sum);
                     }
                 }
             };
@@ -1994,76 +2062,89 @@ __global__ __launch_bounds__(kBlock) void vol_walk_kernel(Params P, const S *__r
                     }
                 }
             };
-            if constexpr (GAUSS) {
-                // ---- one step per piece
-                double t0 = k0, plane[3], next_t[3], unit[3];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const double q = fma(t0, W.B[a], W.A[a]);
-                    const bool moves = inv[a] != 0.0;
-                    unit[a] = W.B[a] >= 0.0 ? 1.0 : -1.0;
-                    plane[a] = unit[a] > 0.0 ? floor(q) + 1.0 : ceil(q) - 1.0;
-                    next_t[a] = moves ? (plane[a] - W.A[a]) * inv[a] : 1e300;
-                    if (next_t[a] <= t0) {
-                        plane[a] += unit[a];
-                        next_t[a] = (plane[a] - W.A[a]) * inv[a];
-                    }
-                }
-                // every step passes a plane or ends the slab; one that does not
-                // advance (planes closer than the rounding of the ray
-                // parameter) flags the view, as in the other kernels of the rule
-                for (int left = P.nx + P.ny + P.nz + 8; t0 < k1 && left > 0; --left) {
-                    const double t1 = fmin(fmin(next_t[0], next_t[1]), fmin(next_t[2], k1));
-                    if (t1 > t0) {
-                        const double radius = 0.5 * (t1 - t0), centre = t0 + radius;
-                        int l[3];
-                        R f[3], b[3];
-#pragma unroll
-                        for (int a = 0; a < 3; ++a) {
-                            walk_split<R>(W.A[a], W.B[a], centre, l[a], f[a]);
-                            b[a] = adv[a];
-                        }
-                        clamp_cell(l, f, b);
-                        deposit(l, f, b, radius * radius * (1.0 / 3.0), 2.0 * (radius * volume_factor));
-                    } else {
-                        bad = true;
-                    }
-#pragma unroll
-                    for (int a = 0; a < 3; ++a)
-                        if (next_t[a] <= t1) {
-                            plane[a] += unit[a];
-                            next_t[a] = (plane[a] - W.A[a]) * inv[a];
-                        }
-                    t0 = fmax(t0, t1);
-                }
-                bad |= t0 < k1;
-            } else {
-                // ---- one step per cell
-                R kf = (R)k0;
-                const R kend = (R)k1;
-                while (kf < kend) {
-                    int l[3];
-                    R f[3], b[3];
-                    R run = (R)1e30;
+            auto march = [&](auto in_brick) {
+                constexpr bool IN_BRICK = decltype(in_brick)::value;
+                // lanes step alone, or (IN_BRICK false) the wave as one
+                const auto more = [](bool left) { return IN_BRICK ? left : __builtin_amdgcn_ballot_w64(left) != 0; };
+                if constexpr (GAUSS) {
+                    // ---- one step per piece
+                    double t0 = k0, plane[3], next_t[3];
+                    const auto unit = [&](int a) { return W.B[a] >= 0.0 ? 1.0 : -1.0; };
 #pragma unroll
                     for (int a = 0; a < 3; ++a) {
-                        walk_split<R>(W.A[a], W.B[a], (double)kf, l[a], f[a]);
-                        // samples until the coordinate leaves [l, l + 1]
-                        run = walk_min(run, walk_fma(-f[a], inv[a], lead[a]));
-                        b[a] = adv[a];
+                        const double q = fma(t0, W.B[a], W.A[a]);
+                        const bool moves = inv[a] != 0.0;
+                        plane[a] = W.B[a] >= 0.0 ? floor(q) + 1.0 : ceil(q) - 1.0;
+                        next_t[a] = moves ? (plane[a] - W.A[a]) * inv[a] : 1e300;
+                        if (next_t[a] <= t0) {
+                            plane[a] += unit(a);
+                            next_t[a] = (plane[a] - W.A[a]) * inv[a];
+                        }
                     }
-                    const R n = walk_min(walk_floor(run) + (R)1, kend - kf);
-                    kf += n;
-                    clamp_cell(l, f, b);
-                    const R half = (R)0.5 * (n - (R)1);
-                    const R var = walk_fma(n * (R)(1.0 / 12.0), n, (R)(-1.0 / 12.0));
+                    // every step passes a plane or ends the slab; one that does not
+                    // advance (planes closer than the rounding of the ray
+                    // parameter) flags the view, as in the other kernels of the rule
+                    for (int left = P.nx + P.ny + P.nz + 8; left > 0 && more(t0 < k1); --left) {
+                        const double t1 = fmin(fmin(next_t[0], next_t[1]), fmin(next_t[2], k1));
+                        const bool live = t0 < k1, ahead = t1 > t0;
+                        bad |= live && !ahead;
+                        if (!IN_BRICK || ahead) {
+                            const double radius = 0.5 * (t1 - t0), centre = t0 + radius;
+                            int l[3];
+                            R f[3], b[3];
 #pragma unroll
-                    for (int a = 0; a < 3; ++a) f[a] = walk_fma(b[a], half, f[a]);
-                    deposit(l, f, b, var, n * (R)volume_factor);
+                            for (int a = 0; a < 3; ++a) {
+                                walk_split<R>(W.A[a], W.B[a], centre, l[a], f[a]);
+                                b[a] = adv[a];
+                            }
+                            clamp_cell(l, f, b);
+                            deposit(in_brick, live && ahead, l, f, b, radius * radius * (1.0 / 3.0),
+                                    2.0 * (radius * volume_factor));
+                        }
+#pragma unroll
+                        for (int a = 0; a < 3; ++a)
+                            if (next_t[a] <= t1) {
+                                plane[a] += unit(a);
+                                next_t[a] = (plane[a] - W.A[a]) * inv[a];
+                            }
+                        t0 = fmax(t0, t1);
+                    }
+                    bad |= t0 < k1;
+                } else {
+                    // ---- one step per cell
+                    R kf = (R)k0;
+                    const R kend = (R)k1;
+                    while (more(kf < kend)) {
+                        const bool live = kf < kend;
+                        int l[3];
+                        R f[3], b[3];
+                        R run = (R)1e30;
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) {
+                            walk_split<R>(W.A[a], W.B[a], (double)kf, l[a], f[a]);
+                            // samples until the coordinate leaves [l, l + 1]
+                            run = walk_min(run, walk_fma(-f[a], inv[a], lead[a]));
+                            b[a] = adv[a];
+                        }
+                        R n = walk_min(walk_floor(run) + (R)1, kend - kf);
+                        if (!IN_BRICK) n = live ? n : (R)0;
+                        kf += n;
+                        clamp_cell(l, f, b);
+                        const R half = (R)0.5 * (n - (R)1);
+                        const R var = walk_fma(n * (R)(1.0 / 12.0), n, (R)(-1.0 / 12.0));
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) f[a] = walk_fma(b[a], half, f[a]);
+                        deposit(in_brick, live, l, f, b, var, n * (R)volume_factor);
+                    }
                 }
+            };
+            if (use_lds) {
+                march(std::true_type{});
+                __syncthreads();
+                walk_drain(P, B, brick, acc);
+            } else {
+                march(std::false_type{});
             }
-            __syncthreads();
-            if (use_lds) walk_drain(P, B, brick, acc);
             __syncthreads();
         }
     }

@@ -3,7 +3,8 @@
 ``vol_walk_kernel`` forms each cell's corner sums in closed form from the
 cell's run of samples: singleton axes and half-cell borders, less than one
 sample per cell, thousands of samples per cell, axes beyond 2^18 grid samples
-(FP64 coordinates instead of biased ones), and slabs that fit no brick.
+(FP64 coordinates instead of biased ones), slabs that fit no brick, and rays
+too sparse for one.
 """
 
 from __future__ import annotations
@@ -52,14 +53,59 @@ def test_cell_sums_match_the_per_sample_scatter(shape, samples, precision):
     assert _rel(actual, expected) <= (1e-5 if precision == "float32" else 1e-7)
 
 
-@pytest.mark.parametrize("cap", ["512", "8192"])
+def _blocky():
+    return O.Grid((40, 44, 48), (1.0, 1.0, 1.0), (-23.5, -21.5, -19.5))
+
+
 @pytest.mark.parametrize("precision", ["float32", "float64"])
-def test_slabs_that_fit_no_brick_use_device_atomics(cap, precision, monkeypatch):
-    print(f"case walk cap={cap} {precision}", flush=True)
-    monkeypatch.setenv("DPT_AMD_BRICK_CAP", cap)
-    grid = O.Grid((40, 44, 48), (1.0, 1.0, 1.0), (-23.5, -21.5, -19.5))
-    actual, expected = _volume(grid, 61, precision, rows=16, cols=16)  # about 4 voxels between pixels
+def test_slabs_that_fit_no_brick_use_device_atomics(precision, monkeypatch):
+    """Dense rays (1.6 voxels apart) whose tiles cover 26 x 26 voxels: a slab of
+    one sample holds more than 512 entries."""
+    print(f"case walk cap=512 {precision}", flush=True)
+    monkeypatch.setenv("DPT_AMD_BRICK_CAP", "512")
+    actual, expected = _volume(_blocky(), 61, precision, rows=40, cols=40)
     assert _rel(actual, expected) <= (1e-5 if precision == "float32" else 1e-7)
+
+
+@pytest.mark.parametrize("views_per_block", ["1", "2", "4"])
+@pytest.mark.parametrize("samples", [1, 7, 61, 900])
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+def test_sparse_rays_add_by_pairs_of_lanes(samples, precision, views_per_block, monkeypatch):
+    """Rays four voxels apart walk without bricks, the wave as one, until its last
+    ray ends."""
+    print(f"case walk sparse S={samples} {precision} vb={views_per_block}", flush=True)
+    monkeypatch.setenv("DPT_AMD_VIEWS_PER_BLOCK", views_per_block)
+    actual, expected = _volume(_blocky(), samples, precision, views=5, rows=16, cols=15)
+    assert _rel(actual, expected) <= (1e-5 if precision == "float32" else 1e-7)
+
+
+@pytest.mark.parametrize("shape", [(1, 44, 48), (40, 1, 48), (40, 44, 1), (40, 44, 48)])
+@pytest.mark.parametrize("mode", ["float32", "float64", "cell_gauss"])
+def test_random_rays_match_the_oracle(shape, mode):
+    """Bundles of random directions, a partial last wave, rays that miss and zero
+    cotangents among them, singleton axes."""
+    print(f"case walk random {shape} {mode}", flush=True)
+    grid = O.Grid(shape, (1.0, 0.9, 1.1), tuple(-0.5 * (n - 1) * h for n, h in zip(shape[::-1], (1.0, 0.9, 1.1))))
+    rng = np.random.default_rng(11)
+    ends = rng.normal(size=(2, 333, 3))
+    ends *= 40.0 / np.linalg.norm(ends, axis=2, keepdims=True)
+    if 1 in shape:  # rays near the plane of the grid
+        ends[..., 2 - shape.index(1)] *= 0.01
+    rays = (ends[0], ends[1])
+    seeds = rng.uniform(-1.0, 1.0, 333)
+    seeds[::7] = 0.0
+    values = np.full(grid.voxels, 0.02, np.float32)
+    precision = "float32" if mode == "float32" else "float64"
+    seeds = seeds.astype(precision)
+    gauss = mode == "cell_gauss"
+    expected, _, _, _ = O.Scene(grid, 97, rays=rays).vjp(values, seeds, precision="fp32" if mode == "float32" else "fp64",
+                                                         pose=False, **(dict(integration=mode) if gauss else {}))
+    gpu = NativeScene(grid, 97, rays=rays, precision=precision, extra_needs=_native.CELL_GAUSS if gauss else 0)
+    actual, _, status = gpu.vjp(values, seeds, pose_grad=False)
+    assert not any(status)
+    assert np.linalg.norm(expected) > 0
+    # the oracle's FP32 positions (|p| <= 40 mm at 2^-24: 2.4e-6 voxel) and FP32 increments
+    assert _rel(actual, expected) <= (1e-5 if mode == "float32" else 1e-7)
 
 
 @pytest.mark.parametrize("precision", ["float32", "float64"])
