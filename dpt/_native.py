@@ -376,9 +376,10 @@ class Plan:
         return value
 
     def layout(self) -> dict:
-        """The launch layout the plan chose (brick entries, slab chunks,
-        samples per chunk, views per VJP workgroup, cell-Gauss chunks per
-        ray)."""
+        """The launch layout the plan chose: brick entries of the volume
+        adjoint, samples in the unit of its sample segments, views per VJP
+        workgroup, first slabs per axis of the cell-Gauss volume adjoint
+        (``slab_chunks`` is always False: every volume adjoint walks slabs)."""
         out = np.zeros(5, dtype=np.int32)
         check(lib().dpt_plan_layout(self.handle, out.ctypes.data), "dpt_plan_layout")
         return {"brick_cap": int(out[0]), "slab_chunks": bool(out[1]), "chunk_samples": int(out[2]),

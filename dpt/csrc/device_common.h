@@ -53,9 +53,7 @@ struct Params {
     const double *ray_end;
     const double *poses;     // views x 12
     int *status;             // views
-    int brick_cap;           // index-chunk brick estimate of the plan (choose_brick_cap)
     int walk_cap;            // FP64 LDS brick entries per workgroup of the volume adjoint
-    int slab_chunks;         // 1: index chunks would overflow even the larger brick often (silhouette-heavy plans)
     int chunk_samples;       // unit of the sample segments
     int gauss_chunks;        // first slabs per axis of the cell-Gauss volume adjoint
     const double *alpha64;   // 2 x samples entries (FP64 sampling): (k + 0.5) / S, then 1 - that

@@ -163,8 +163,8 @@ __device__ __forceinline__ void store_gradient(const Params &P, const double *g,
     }
 }
 
-// Brick = axis-aligned box of grid samples that one workgroup's rays touch
-// during one chunk of samples, privatised in LDS.
+// Brick = axis-aligned box of grid samples that one workgroup's rays touch in
+// one slab, privatised in LDS.
 struct Brick {
     int x0, y0, z0;      // first sample of the box
     int bx, by, bz;      // extents
@@ -189,180 +189,16 @@ inline int chunk_samples(int samples, int nx, int ny, int nz) {
     const double chunk = 32.0 * samples / 1024.0 * 443.4 / diagonal;
     return (int)std::lround(std::fmin(64.0, std::fmax(8.0, chunk)));
 }
-// Brick entries that choose_brick_cap reports (dpt_plan_layout).  gfx950
-// executes ds_add_f64 about ten times faster than ds_add_f32 (16.5 against 193
-// cycles per wave64 instruction at brick addresses, measured), so bricks
-// accumulate in FP64.
-constexpr int kBrickCapDefault = 4096;
 
-// Host estimate of the chunk bricks at the identity pose, from up to four
-// views spread over the scan (views 0, V/4, V/2, 3V/4): the grid samples
-// touched by 16 x 16 pixel tiles (every 4th tile along each detector axis,
-// at most 16 per axis) over one chunk of samples at a quarter, half and three
-// quarters of the ray.  The counts of all sampled views are pooled.  A plan takes bricks of
-// 2 * kBrickCapDefault FP64 entries (64 KiB of LDS, fewer workgroups per CU)
-// only when at least a quarter of the sampled bricks overflow
-// kBrickCapDefault yet fit the larger brick: magnified detectors over fine
-// grids, whose tiles cover wide footprints and would otherwise fall back to
-// device atomics.  (A 256^3 grid under a 512^2 panel at 1.5x magnification
-// overflows in 9 % of the samples and keeps the default; a 512 x 512 x 139
-// chest grid at 0.76 mm under a 512^2 panel at 2.67 mm overflows in 60 %.)
-// *slab_chunks reports a silhouette-heavy plan: its tiles overflow even the
-// larger brick often by index chunks and rarely by slabs of space (the chest
-// grid: in 15 % of the index chunks and in none of the slab chunks).
-int choose_brick_cap(const Params &P, const double *panels, int *slab_chunks) {
-    const int n[3] = {P.nx, P.ny, P.nz};
-    const int chunks = (P.samples + P.chunk_samples - 1) / P.chunk_samples;
-    const int tile = 16;
-    const int tiles_y = (P.rows + tile - 1) / tile, tiles_x = (P.cols + tile - 1) / tile;
-    const int step_y = std::max(4, (tiles_y + 15) / 16), step_x = std::max(4, (tiles_x + 15) / 16);
-    const int sampled_chunks[3] = {chunks / 4, chunks / 2, (3 * chunks) / 4};
-    int measured = 0, rescued = 0, index_over = 0, slab_measured = 0, slab_over = 0;  // over: > 2 * default
-    const int sampled_views = std::min(P.views, 4);
-    for (int sv = 0; sv < sampled_views; ++sv)
-    for (int ty = 0; ty < tiles_y; ty += step_y)
-        for (int tx = 0; tx < tiles_x; tx += step_x) {
-            const double *pv = panels + 12 * (size_t)((long long)sv * P.views / sampled_views);
-            // the tile's rays in grid coordinates with their clipped intervals
-            struct TileRay {
-                double o[3], d[3], t0, step;
-            };
-            std::vector<TileRay> rays;
-            for (int r = ty * tile; r < std::min(ty * tile + tile, P.rows); ++r)
-                for (int c = tx * tile; c < std::min(tx * tile + tile, P.cols); ++c) {
-                    TileRay tr;
-                    double src[3], end[3];
-                    for (int a = 0; a < 3; ++a) {
-                        src[a] = pv[a] - P.go[a];
-                        end[a] = pv[3 + a] + c * pv[6 + a] + r * pv[9 + a] - pv[a];
-                    }
-                    for (int a = 0; a < 3; ++a) {
-                        tr.o[a] = P.g[3 * a] * src[0] + P.g[3 * a + 1] * src[1] + P.g[3 * a + 2] * src[2];
-                        tr.d[a] = P.g[3 * a] * end[0] + P.g[3 * a + 1] * end[1] + P.g[3 * a + 2] * end[2];
-                    }
-                    double t0 = 0.0, t1 = 1.0;
-                    for (int a = 0; a < 3; ++a) {
-                        if (tr.d[a] == 0.0) {
-                            if (tr.o[a] < -0.5 || tr.o[a] > n[a] - 0.5) t1 = -1.0;
-                            continue;
-                        }
-                        const double u = (-0.5 - tr.o[a]) / tr.d[a], v = (n[a] - 0.5 - tr.o[a]) / tr.d[a];
-                        t0 = std::max(t0, std::min(u, v));
-                        t1 = std::min(t1, std::max(u, v));
-                    }
-                    if (!(t1 > t0)) continue;
-                    tr.t0 = t0;
-                    tr.step = (t1 - t0) / P.samples;
-                    rays.push_back(tr);
-                }
-            if (rays.empty()) continue;
-            // slab chunks (the device's slab_setup / slab_range, in FP64 on the host)
-            int votes[3] = {0, 0, 0};
-            for (const TileRay &tr : rays) {
-                const double ad[3] = {std::fabs(tr.d[0]), std::fabs(tr.d[1]), std::fabs(tr.d[2])};
-                ++votes[ad[0] >= ad[1] && ad[0] >= ad[2] ? 0 : (ad[1] >= ad[2] ? 1 : 2)];
-            }
-            const int A = votes[0] >= votes[1] && votes[0] >= votes[2] ? 0 : (votes[1] >= votes[2] ? 1 : 2);
-            int slo = INT_MAX, shi = INT_MIN, adv = 1;
-            for (const TileRay &tr : rays) {
-                const double q0 = tr.o[A] + (tr.t0 + 0.5 * tr.step) * tr.d[A];
-                const double q1 = tr.o[A] + (tr.t0 + (P.samples - 0.5) * tr.step) * tr.d[A];
-                slo = std::min(slo, (int)std::floor(std::min(std::max(std::min(q0, q1), -2.0), n[A] + 1.0)));
-                shi = std::max(shi, (int)std::ceil(std::min(std::max(std::max(q0, q1), -2.0), n[A] + 1.0)));
-                adv = std::max(adv, (int)std::min(std::ceil(tr.step * std::fabs(tr.d[A]) * 64.0), 1048576.0));
-            }
-            const int width = std::max(1, (P.chunk_samples * adv + 63) / 64);
-            const int count = std::max(1, (shi - slo + width - 1) / width);
-            for (int j : {count / 4, count / 2, (3 * count) / 4}) {
-                int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
-                for (const TileRay &tr : rays) {
-                    const double da = tr.d[A];
-                    if (da == 0.0) continue;
-                    const int js = da > 0.0 ? j : count - 1 - j;
-                    const double b0 = slo + js * width, b1 = slo + (js + 1) * width;
-                    const double t0 = ((b0 - tr.o[A]) / da - tr.t0) / tr.step - 0.5;
-                    const double t1 = ((b1 - tr.o[A]) / da - tr.t0) / tr.step - 0.5;
-                    double k0, k1;
-                    if (da > 0.0) {
-                        k0 = j == 0 ? 0.0 : std::min(std::max(std::ceil(t0), 0.0), (double)P.samples);
-                        k1 = j == count - 1 ? P.samples : std::min(std::max(std::ceil(t1), 0.0), (double)P.samples);
-                    } else {
-                        k0 = j == 0 ? 0.0 : std::min(std::max(std::floor(t1) + 1.0, 0.0), (double)P.samples);
-                        k1 = j == count - 1 ? P.samples : std::min(std::max(std::floor(t0) + 1.0, 0.0), (double)P.samples);
-                    }
-                    if (!(k1 > k0)) continue;
-                    for (double k : {k0, k1 - 1.0}) {
-                        const double pos = tr.t0 + (k + 0.5) * tr.step;
-                        for (int a = 0; a < 3; ++a) {
-                            const double x = std::min(std::max(tr.o[a] + pos * tr.d[a], 0.0), (double)(n[a] - 1));
-                            const int l = std::min((int)std::floor(x), std::max(n[a] - 2, 0));
-                            lo[a] = std::min(lo[a], l);
-                            hi[a] = std::max(hi[a], l);
-                        }
-                    }
-                }
-                if (lo[0] == INT_MAX) continue;
-                long long volume = 1;
-                for (int a = 0; a < 3; ++a) volume *= std::min(hi[a] + 1, n[a] - 1) - lo[a] + 1;
-                ++slab_measured;
-                slab_over += volume > 2 * kBrickCapDefault;
-            }
-            for (int q = 0; q < 3; ++q) {
-                const int k0 = sampled_chunks[q] * P.chunk_samples, k1 = std::min(k0 + P.chunk_samples, P.samples);
-                int lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
-                for (int r = ty * tile; r < std::min(ty * tile + tile, P.rows); ++r)
-                    for (int c = tx * tile; c < std::min(tx * tile + tile, P.cols); ++c) {
-                        double src[3], end[3], o[3], d[3];
-                        for (int a = 0; a < 3; ++a) {
-                            src[a] = pv[a] - P.go[a];
-                            end[a] = pv[3 + a] + c * pv[6 + a] + r * pv[9 + a] - pv[a];
-                        }
-                        for (int a = 0; a < 3; ++a) {
-                            o[a] = P.g[3 * a] * src[0] + P.g[3 * a + 1] * src[1] + P.g[3 * a + 2] * src[2];
-                            d[a] = P.g[3 * a] * end[0] + P.g[3 * a + 1] * end[1] + P.g[3 * a + 2] * end[2];
-                        }
-                        double t0 = 0.0, t1 = 1.0;
-                        for (int a = 0; a < 3; ++a) {
-                            if (d[a] == 0.0) {
-                                if (o[a] < -0.5 || o[a] > n[a] - 0.5) t1 = -1.0;
-                                continue;
-                            }
-                            const double u = (-0.5 - o[a]) / d[a], v = (n[a] - 0.5 - o[a]) / d[a];
-                            t0 = std::max(t0, std::min(u, v));
-                            t1 = std::min(t1, std::max(u, v));
-                        }
-                        if (!(t1 > t0)) continue;
-                        const double step = (t1 - t0) / P.samples;
-                        for (int k : {k0, k1 - 1}) {
-                            const double pos = t0 + (k + 0.5) * step;
-                            for (int a = 0; a < 3; ++a) {
-                                const double x = std::min(std::max(o[a] + pos * d[a], 0.0), (double)(n[a] - 1));
-                                const int l = std::min((int)std::floor(x), std::max(n[a] - 2, 0));
-                                lo[a] = std::min(lo[a], l);
-                                hi[a] = std::max(hi[a], l);
-                            }
-                        }
-                    }
-                if (lo[0] == INT_MAX) continue;
-                long long volume = 1;
-                for (int a = 0; a < 3; ++a) volume *= std::min(hi[a] + 1, n[a] - 1) - lo[a] + 1;
-                ++measured;
-                rescued += volume > kBrickCapDefault && volume <= 2 * kBrickCapDefault;
-                index_over += volume > 2 * kBrickCapDefault;
-            }
-        }
-    *slab_chunks = measured > 0 && slab_measured > 0 && 16 * index_over >= measured &&
-                   2 * slab_over * measured < index_over * slab_measured;
-    if (*slab_chunks) return 2 * kBrickCapDefault;
-    return measured > 0 && 4 * rescued >= measured ? 2 * kBrickCapDefault : kBrickCapDefault;
-}
-
-// Bound one chunk's cells over the workgroup and, when the box fits the LDS
-// brick, describe it; e: the box's extents in grid samples.  lo / nhi: this lane's lower cell corner minimum and
-// negated maximum over its chunk samples (INT_MAX when it has none).  Every
-// lane gets the same answer (kept in SGPRs); one barrier.
+// Bound one slab's cells over the workgroup and, when the box fits the LDS
+// brick of `cap` FP64 entries, describe it; e: the box's extents in grid samples.
+// lo / nhi: this lane's lower cell corner minimum and negated maximum over its
+// samples in the slab (INT_MAX when it has none).  Every lane gets the same
+// answer (kept in SGPRs); one barrier.  gfx950 executes ds_add_f64 about ten
+// times faster than ds_add_f32 (16.5 against 193 cycles per wave64 instruction at
+// brick addresses, measured), so bricks accumulate in FP64.
 __device__ __forceinline__ bool chunk_brick(const Params &P, int (*red)[6], int *lo, int *nhi, int cap, bool unit_x,
-                                            Brick &B, bool pad, int *e) {
+                                            Brick &B, int *e) {
     const int wv = threadIdx.x >> 6;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -393,16 +229,15 @@ __device__ __forceinline__ bool chunk_brick(const Params &P, int (*red)[6], int 
     B.x0 = __builtin_amdgcn_readfirstlane(l[0]);
     B.y0 = __builtin_amdgcn_readfirstlane(l[1]);
     B.z0 = __builtin_amdgcn_readfirstlane(l[2]);
-    // pad: odd row and plane strides when the padded box still fits (FP64
-    // entries whose indices differ by a multiple of 32 share an LDS bank, so
-    // even strides line up the corners of neighbouring rays' cells).  Only
-    // for callers that write cells inside the bound box: the padding stays
-    // zero and the drain skips it.
+    // odd row and plane strides when the padded box still fits (FP64 entries
+    // whose indices differ by a multiple of 32 share an LDS bank, so even
+    // strides line up the corners of neighbouring rays' cells); the padding
+    // stays zero and the drain skips it
     int px = e[0], py = e[1];
-    // Padded strides keep flush_lds's global-coordinate index below 2^24 per
-    // operand and 2^31 overall when nz (ny + 1) and nz (ny + 1) (nx + 1) do.
+    // Padded strides keep the walk's global-coordinate index of a corner below
+    // 2^24 per operand and 2^31 overall when nz (ny + 1) and nz (ny + 1) (nx + 1) do.
     const long long plane = (long long)P.nz * (P.ny + 1);
-    if (pad && (long long)(px | 1) * (py | 1) * e[2] <= cap && plane <= (1 << 24) &&
+    if ((long long)(px | 1) * (py | 1) * e[2] <= cap && plane <= (1 << 24) &&
         plane * (P.nx + 1) <= INT_MAX)
         px |= 1, py |= 1;
     B.bx = __builtin_amdgcn_readfirstlane(px);
@@ -1547,30 +1382,30 @@ __global__ __launch_bounds__(kBlock, 3) void vjp_gauss_kernel(Params P, const T 
                 break;
             }
             bad |= !finite3d(s.first) || !finite3d(s.second);
-                double g1[3], g2[3], v1, v2;
-                if (s.shared) {  // one load of the cell for both nodes
-                    double v[8];
-                    load8d<T>(P, field, (s.lower[2] * P.ny + s.lower[1]) * P.nx + s.lower[0], v);
-                    v1 = node_in_cell<true>(P, s.first, s.lower, v, g1);
-                    v2 = node_in_cell<true>(P, s.second, s.lower, v, g2);
-                } else {
-                    v1 = node_value<T, true>(P, field, s.first, nullptr, g1);
-                    v2 = node_value<T, true>(P, field, s.second, nullptr, g2);
-                }
-                if constexpr (C == kRayCoordinates) {
-                    integral += s.radius * v1;
-                    integral += s.radius * v2;
-                }
+            double g1[3], g2[3], v1, v2;
+            if (s.shared) {  // one load of the cell for both nodes
+                double v[8];
+                load8d<T>(P, field, (s.lower[2] * P.ny + s.lower[1]) * P.nx + s.lower[0], v);
+                v1 = node_in_cell<true>(P, s.first, s.lower, v, g1);
+                v2 = node_in_cell<true>(P, s.second, s.lower, v, g2);
+            } else {
+                v1 = node_value<T, true>(P, field, s.first, nullptr, g1);
+                v2 = node_value<T, true>(P, field, s.second, nullptr, g2);
+            }
+            if constexpr (C == kRayCoordinates) {
+                integral += s.radius * v1;
+                integral += s.radius * v2;
+            }
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    og[a] += s.radius * g1[a];
-                    og[a] += s.radius * g2[a];
-                }
+            for (int a = 0; a < 3; ++a) {
+                og[a] += s.radius * g1[a];
+                og[a] += s.radius * g2[a];
+            }
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    dg[a] += s.radius * s.first_position * g1[a];
-                    dg[a] += s.radius * s.second_position * g2[a];
-                }
+            for (int a = 0; a < 3; ++a) {
+                dg[a] += s.radius * s.first_position * g1[a];
+                dg[a] += s.radius * s.second_position * g2[a];
+            }
             start = s.end;
             advance_cells(P, r, walk, s.end, iv.upper);
         }
@@ -1958,7 +1793,7 @@ __global__ __launch_bounds__(kBlock, (std::is_same<R, float>::value ? 6 : 4)) vo
             __syncthreads();  // the bound rewrites bound_red
             if (lane == 0) ray_red[wv] = rays;
             Brick B{};
-            (void)chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, true, e);
+            (void)chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, e);
             const float across = axis == 0 ? (float)e[1] * e[2] : (axis == 1 ? (float)e[0] * e[2] : (float)e[0] * e[1]);
             const bool sparse = (float)(ray_red[0] + ray_red[1] + ray_red[2] + ray_red[3]) < kWalkSparse * across;
             return (bool)__builtin_amdgcn_readfirstlane(sparse);
@@ -1982,7 +1817,7 @@ __global__ __launch_bounds__(kBlock, (std::is_same<R, float>::value ? 6 : 4)) vo
                 if (sparse) break;
                 int blo[3], bnhi[3], e[3];
                 cell_bounds(k0, k1, GAUSS, blo, bnhi);
-                use_lds = chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, true, e);
+                use_lds = chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, e);
                 box = (long long)e[0] * e[1] * e[2];
                 if (box <= P.walk_cap || s1 - s0 <= 1) break;
                 width = max(1, (s1 - s0) >> 1);
@@ -2626,10 +2461,14 @@ int choose_views_per_block(const double *panels, int views, int rows, int cols) 
 
 // FP64 LDS brick entries per workgroup of the volume adjoint (vol_walk_kernel):
 // the least multiple of 512 that holds a slab of kWalkWidth grid samples for
-// half of the sampled tiles at the identity pose.  Smaller bricks leave more workgroups
-// on a CU, larger ones fewer and wider slabs: the full scan runs 206 / 213 /
-// 229 ms at 2048 / 4096 / 8192 entries, 60 views of 256^2 over 128^3 4.5 / 3.9
-// / 4.5, 24 views of 256^2 over 256^3 27 / 15.5 / 11.6.
+// half of the sampled tiles at the identity pose.  Smaller bricks leave more
+// workgroups on a CU, larger ones fewer and wider slabs: the volume adjoint takes
+// 62 / 68 / 78 ms at 2048 / 4096 / 8192 entries on the full scan (rule: 2048),
+// 2.3 / 2.1 / 2.7 for 60 views of 256^2 over 128^3 (3072: 2.0), 17.6 / 10.2 / 5.7
+// for 24 views over 256^3 (8192).  Explicit rays and panel records take 8192
+// (kWalkCapMost): 24 parallel views of 256^2 over 128^3 1.76 / 1.37 / 1.31 ms, 24
+// cylindrical ones 3.9 / 2.2 / 1.7; an ordered bundle of 512^2 rays over 256^3
+// would do better with less, 0.74 / 0.73 / 0.90.
 constexpr int kWalkCapLeast = 2048, kWalkCapMost = 8192;
 int choose_walk_cap(const Params &base, const double *panels, int vb) {
     Params P = base;
@@ -3001,16 +2840,10 @@ int plan_create(const dpt_grid_desc *grid, int32_t views, int32_t rows, int32_t 
         const int forced = std::atoi(chunks);
         if (forced >= 1 && forced <= 256) P.gauss_chunks = forced;
     }
-    P.slab_chunks = 0;
-    P.brick_cap = P.bundle ? kBrickCapDefault : choose_brick_cap(P, panels, &P.slab_chunks);
     P.walk_cap = P.bundle ? kWalkCapMost : choose_walk_cap(P, panels, choose_views_per_block(panels, views, rows, cols));
     if (const char *cap = std::getenv("DPT_AMD_BRICK_CAP")) {
         const int forced = std::atoi(cap);
-        if (forced >= 512 && forced <= 8192) P.brick_cap = P.walk_cap = forced;
-    }
-    if (const char *slab = std::getenv("DPT_AMD_SLAB_CHUNKS")) {
-        if (std::strcmp(slab, "0") == 0) P.slab_chunks = 0;
-        if (std::strcmp(slab, "1") == 0) P.slab_chunks = 1;
+        if (forced >= 512 && forced <= 8192) P.walk_cap = forced;
     }
     p->vjp_vb = P.bundle ? 1 : choose_views_per_block(panels, views, rows, cols);
     if (const char *vb = std::getenv("DPT_AMD_VIEWS_PER_BLOCK")) {
@@ -3496,8 +3329,8 @@ int dpt_adjoint_gather_noalloc(dpt_plan *p, const double *poses, const double *c
 
 int dpt_plan_layout(const dpt_plan *p, int32_t *out) {
     if (p == nullptr || out == nullptr) return fail(DPT_E_INVALID, "plan and out are required");
-    out[0] = p->base.brick_cap;
-    out[1] = p->base.slab_chunks;
+    out[0] = p->base.walk_cap;
+    out[1] = 0;
     out[2] = p->base.chunk_samples;
     out[3] = p->vjp_vb;
     out[4] = p->base.gauss_chunks;

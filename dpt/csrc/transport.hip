@@ -683,7 +683,8 @@ __global__ void zero_counter_kernel(unsigned long long *counter) { *counter = 0u
 // Lanes that wait for an ended photon's score or a new photon before the wave
 // stops for them.  A wave ran both at every event, for one lane in twelve:
 // 10^7 histories of the 40-120 keV spectrum on 128^3 take 7.29 / 7.04 / 6.54 /
-// 6.48 / 6.66 ms at 1 / 8 / 16 / 24 / 32.
+// 6.48 / 6.66 ms at 1 / 8 / 16 / 24 / 32; 5e6 at 60 keV on 96^3 3.02 / 2.79 / 2.77
+// / 2.79 / 2.97 at 8 / 14 / 20 / 28 / 40, on 48^3 1.93 / 1.91 / 1.82 / 1.82 / 1.87.
 constexpr int kRefill = 20;
 
 // Three waves per SIMD: 168 VGPRs and 112 bytes of spills.  Four spill 264

@@ -306,12 +306,11 @@ int dpt_compose_pose(const double *anchor, const double *tangent, int64_t count,
 int dpt_compose_pose_vjp(const double *anchor, const double *jet, const double *grad_out, int64_t count,
                          double *grad_anchor, double *grad_tangent, void *stream);
 
-/* The launch layout a plan chose: out[0] FP64 LDS brick entries of the
- * volume adjoint, out[1] 1 when the FP64 volume adjoint chunks by slabs of
- * grid samples instead of runs of sample indices, out[2] samples per chunk,
- * out[3] views per workgroup of the VJP launches, out[4] chunks per ray of
- * the cell-Gauss volume adjoint.  Inspection helper, no reference
- * counterpart. */
+/* The launch layout a plan chose: out[0] FP64 LDS brick entries per workgroup
+ * of the volume adjoint, out[1] 0 (reserved), out[2] samples in the unit of the
+ * volume adjoint's sample segments, out[3] views per workgroup of the VJP
+ * launches, out[4] first slabs per axis of the cell-Gauss volume adjoint.
+ * Inspection helper, no reference counterpart. */
 int dpt_plan_layout(const dpt_plan *plan, int32_t *out);
 
 const char *dpt_last_error(void);

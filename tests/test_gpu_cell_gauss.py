@@ -79,10 +79,10 @@ def test_cell_gauss_vjp_matches_the_oracle(name, components):
 @pytest.mark.parametrize("cap,chunks", [(None, None), ("512", "1"), ("512", "64"), (None, "1"), (None, "64"),
                                         ("8192", "3")])
 def test_cell_gauss_volume_bricks_match_the_oracle(cap, chunks, mode, monkeypatch):
-    """The volume adjoint's lockstep chunks and LDS bricks: the plan's own
-    chunking, one chunk per ray, 64 chunks (shorter than a cell), the largest
-    brick, and the smallest (512 entries), where chunks overflow, are halved
-    and at 1/8 add to the device accumulator."""
+    """The volume adjoint's slabs and LDS bricks: the plan's own first slabs, one
+    an axis, 64 an axis (thinner than a cell), the largest brick, and the
+    smallest (512 entries), where slabs overflow, are halved and in the end add
+    to the device accumulator."""
     print(f"case cell-gauss bricks cap={cap} chunks={chunks} {mode}", flush=True)
     if cap is not None:
         monkeypatch.setenv("DPT_AMD_BRICK_CAP", cap)

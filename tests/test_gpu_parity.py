@@ -171,10 +171,10 @@ def test_fp32_vjp_matches_oracle(name, mode, components):
 def test_fp32_vjp_sample_segments(name, segments, cells, monkeypatch):
     """Launches of few tiles split each tile's samples into segments (by
     default here: 1024 samples, 256 per segment) for the volume adjoint; the
-    pose adjoint of FP32 storage runs those launches unsegmented through the
-    pipelined sample loop, so each ray's pose sums are the oracle's one
-    sequential FP32 sum: the pose gradient agrees up to the FP64 order of the
-    cross-ray sums, joint and pose-only, linear and cell gathers."""
+    pose adjoint of those launches adds each ray in one wave, so its pose sums
+    are the oracle's one sequential FP32 sum: the pose gradient agrees up to the
+    FP64 order of the cross-ray sums, joint and pose-only, linear and copied
+    gathers."""
     print(f"case segments {name} {segments} cells={cells}", flush=True)
     if segments is not None:
         monkeypatch.setenv("DPT_AMD_VJP_SEGMENTS", segments)
@@ -190,154 +190,70 @@ def test_fp32_vjp_sample_segments(name, segments, cells, monkeypatch):
         assert _rel(p_gpu, p_ref) <= 1e-12, (vol, _rel(p_gpu, p_ref))
 
 
-def test_half_storage_pose_segments_stay_near_the_fp64_vjp(monkeypatch):
-    """16-bit storage segments the pose too (its blocked compensated sums have
-    no sequential FP32 counterpart): against the FP64 VJP of the rounded field
-    it stays as close as the unsegmented launch, and as the oracle's FP32 VJP
-    of that field."""
-    print("case half segments", flush=True)
-    grid, values, pose, ref, _ = _scene("cone", 1024, storage="bfloat16")
-    rounded = torch.tensor(values, dtype=torch.float32).to(torch.bfloat16).float().numpy()
+@pytest.mark.parametrize("cap,segments", [(None, "1"), (None, "4"), ("512", None)])
+@pytest.mark.parametrize("storage", ["bfloat16", "float16"])
+def test_half_storage_gradients_match_the_oracle_on_the_rounded_field(storage, cap, segments, monkeypatch):
+    """16-bit storage, joint: the volume gradient (which does not read the field)
+    against the oracle's FP32 VJP, with one and four sample segments and with
+    bricks that overflow; the pose gradient (blocked compensated sums, which have
+    no sequential FP32 counterpart) as close to the FP64 VJP of the rounded field
+    as the oracle's FP32 VJP of that field is."""
+    print(f"case half {storage} cap={cap} segments={segments}", flush=True)
+    for name, value in (("DPT_AMD_BRICK_CAP", cap), ("DPT_AMD_VJP_SEGMENTS", segments)):
+        if value is not None:
+            monkeypatch.setenv(name, value)
+    grid, values, pose, ref, gpu = _scene("cone", 1024, storage=storage)
+    dtype = torch.bfloat16 if storage == "bfloat16" else torch.float16
+    rounded = torch.tensor(values, dtype=torch.float32).to(dtype).float().numpy()
     image, _ = ref.forward(rounded, pose)
     seeds = np.random.default_rng(31).uniform(-1.0, 1.0, image.size).astype(np.float32)
     _, p64, _, _ = ref.vjp(rounded, seeds.astype(np.float64), pose, precision="fp64", volume=False)
-    _, p32, _, _ = ref.vjp(rounded, seeds, pose, volume=False)
-    errors = []
-    for segments in ("1", "4"):
-        monkeypatch.setenv("DPT_AMD_VJP_SEGMENTS", segments)
-        *_, gpu = _scene("cone", 1024, storage="bfloat16")
-        _, p_gpu, status = gpu.vjp(values, seeds, pose, volume=False)
-        assert status.tolist() == [0] * len(status)
-        errors.append(_rel(p_gpu, p64))
-    assert errors[1] <= 1.5 * errors[0] + 1e-7, errors
-    assert max(errors) <= 1.5 * _rel(p32, p64) + 1e-7, (errors, _rel(p32, p64))
+    g32, p32, _, _ = ref.vjp(rounded, seeds, pose)
+    g_gpu, p_gpu, status = gpu.vjp(values, seeds, pose)
+    assert status.tolist() == [0] * len(status)
+    assert _rel(g_gpu, g32) <= 1e-5
+    assert _rel(p_gpu, p64) <= 1.5 * _rel(p32, p64) + 1e-7
 
 
-@pytest.mark.parametrize("fallback", ["1", "0"])
 @pytest.mark.parametrize("precision", ["float32", "float64"])
-@pytest.mark.parametrize("cap,chunk", [("512", None), ("512", "7"), (None, "1"), (None, "64"), ("8192", "16")])
-def test_volume_vjp_brick_paths_match_oracle(cap, chunk, precision, fallback, monkeypatch):
-    """LDS bricks of every size down to the smallest capacity (512 entries),
-    where most chunks overflow: the FP32 kernel then walks the rest of the
-    workgroup's samples by slab chunks (fallback "1", the default) or flushes
-    the chunk to device atomics ("0"); chunk lengths from 1 to 64 samples.
-    The pose sums keep their order either way."""
-    print(f"case bricks cap={cap} chunk={chunk} {precision} fallback={fallback}", flush=True)
-    monkeypatch.setenv("DPT_AMD_SLAB_FALLBACK", fallback)
-    if cap is not None:
-        monkeypatch.setenv("DPT_AMD_BRICK_CAP", cap)
-    if chunk is not None:
-        monkeypatch.setenv("DPT_AMD_CHUNK", chunk)
+@pytest.mark.parametrize("cap,segments,chunk", [("512", None, None), ("512", "3", "7"), (None, "2", "1"),
+                                                (None, "4", "16"), ("1024", None, None), ("8192", None, None)])
+def test_volume_vjp_brick_paths_match_oracle(cap, segments, chunk, precision, monkeypatch):
+    """LDS bricks from the smallest capacity (512 entries), where slabs are halved
+    until they fit or go to device atomics, to the largest, and sample segments
+    of 1 to 16 samples' units; joint and volume-only.  The pose sums keep their
+    order throughout."""
+    print(f"case bricks cap={cap} segments={segments} chunk={chunk} {precision}", flush=True)
+    for name, value in (("DPT_AMD_BRICK_CAP", cap), ("DPT_AMD_VJP_SEGMENTS", segments), ("DPT_AMD_CHUNK", chunk)):
+        if value is not None:
+            monkeypatch.setenv(name, value)
     grid, panels, values = _cone(n=24, views=5, rows=20, cols=28, seed=4)
     pose = scenes.compose(scenes.IDENTITY12, (0.5, -0.7, 0.3, 0.02, -0.015, 0.03))
     ref = O.Scene(grid, 97, panels=panels)
     gpu = NativeScene(grid, 97, panels=panels, precision=precision)
+    if cap is not None:
+        assert gpu.plan.layout()["brick_cap"] == int(cap)
     fp = "fp32" if precision == "float32" else "fp64"
     image, _ = ref.forward(values, pose, precision=fp)
     seeds = np.random.default_rng(8).uniform(-1.0, 1.0, image.size)
     if precision == "float32":
         seeds = seeds.astype(np.float32)
     g_ref, p_ref, _, _ = ref.vjp(values, seeds, pose, precision=fp)
-    g_gpu, p_gpu, status = gpu.vjp(values, seeds, pose)
-    assert status.tolist() == [0] * len(status)
-    assert _rel(g_gpu, g_ref) <= (1e-5 if precision == "float32" else 1e-7)
-    # FP32: each ray's pose sums are the oracle's sequential FP32 sums
-    assert _rel(p_gpu, p_ref) <= (1e-12 if precision == "float32" else 1e-10)
-    if precision == "float32":
-        g_vol, _, status = gpu.vjp(values, seeds, pose, pose_grad=False)
-        assert status.tolist() == [0] * len(status)
-        assert _rel(g_vol, g_ref) <= 1e-5
-
-
-@pytest.mark.parametrize("storage", ["bfloat16", "float16"])
-def test_half_storage_slab_fallback_matches_index_chunks(storage, monkeypatch):
-    """16-bit storage (blocked compensated pose sums) through the slab
-    fallback: with the smallest brick most workgroups switch to slab chunks,
-    whose compensation blocks differ from the index chunks' (device-atomic
-    flushes); volume and pose gradients agree to FP32 rounding."""
-    print(f"case half slab fallback {storage}", flush=True)
-    monkeypatch.setenv("DPT_AMD_BRICK_CAP", "512")
-    grid, panels, values = _cone(n=24, views=5, rows=20, cols=28, seed=5)
-    pose = scenes.compose(scenes.IDENTITY12, (0.5, -0.7, 0.3, 0.02, -0.015, 0.03))
-    ref = O.Scene(grid, 97, panels=panels)
-    image, _ = ref.forward(values, pose)
-    seeds = np.random.default_rng(9).uniform(-1.0, 1.0, image.size).astype(np.float32)
-    out = {}
-    for fallback in ("1", "0"):
-        monkeypatch.setenv("DPT_AMD_SLAB_FALLBACK", fallback)
-        gpu = NativeScene(grid, 97, panels=panels, storage=storage)
-        g, p_, status = gpu.vjp(values, seeds, pose)
-        assert status.tolist() == [0] * len(status)
-        out[fallback] = (g, p_)
-    assert _rel(out["1"][0], out["0"][0]) <= 1e-6
-    assert _rel(out["1"][1], out["0"][1]) <= 1e-6
-
-
-@pytest.mark.parametrize("mode", ["both", "volume"])
-@pytest.mark.parametrize("cap,chunk", [(None, None), ("512", None), (None, "1"), ("512", "7"), (None, "64")])
-def test_fp64_slab_chunks_match_oracle(cap, chunk, mode, monkeypatch):
-    """The FP64 volume adjoint chunked by slabs of grid samples (forced on),
-    joint and volume-only, from the smallest brick (device-atomic fallback
-    chunks) up, chunk lengths 1 to 64."""
-    print(f"case slabs cap={cap} chunk={chunk} {mode}", flush=True)
-    monkeypatch.setenv("DPT_AMD_SLAB_CHUNKS", "1")
-    if cap is not None:
-        monkeypatch.setenv("DPT_AMD_BRICK_CAP", cap)
-    if chunk is not None:
-        monkeypatch.setenv("DPT_AMD_CHUNK", chunk)
-    grid, panels, values = _cone(n=24, views=5, rows=20, cols=28, seed=6)
-    pose = scenes.compose(scenes.IDENTITY12, (0.5, -0.7, 0.3, 0.02, -0.015, 0.03))
-    ref = O.Scene(grid, 97, panels=panels)
-    gpu = NativeScene(grid, 97, panels=panels, precision="float64")
-    assert gpu.plan.layout()["slab_chunks"]
-    image, _ = ref.forward(values, pose, precision="fp64")
-    seeds = np.random.default_rng(12).uniform(-1.0, 1.0, image.size)
-    pose_grad = mode == "both"
-    g_ref, p_ref, _, _ = ref.vjp(values, seeds, pose, precision="fp64", pose=pose_grad)
-    g_gpu, p_gpu, status = gpu.vjp(values, seeds, pose, pose_grad=pose_grad)
-    assert status.tolist() == [0] * len(status)
-    assert _rel(g_gpu, g_ref) <= 1e-7
-    if pose_grad:
-        assert _rel(p_gpu, p_ref) <= 1e-10
-
-
-@pytest.mark.parametrize("segments", [None, "1", "4"])
-@pytest.mark.parametrize("cap,chunk", [(None, None), ("512", None), (None, "1"), ("512", "7"), (None, "64")])
-def test_fp32_slab_chunks_match_oracle(cap, chunk, segments, monkeypatch):
-    """The FP32 volume adjoint chunked by slabs of grid samples (forced on):
-    volume-only and, where the launch segments, beside the pipelined pose
-    adjoint; from the smallest brick (device-atomic fallback chunks) up,
-    chunk lengths 1 to 64, one to four sample segments."""
-    print(f"case fp32 slabs cap={cap} chunk={chunk} segments={segments}", flush=True)
-    monkeypatch.setenv("DPT_AMD_SLAB_CHUNKS", "1")
-    if cap is not None:
-        monkeypatch.setenv("DPT_AMD_BRICK_CAP", cap)
-    if chunk is not None:
-        monkeypatch.setenv("DPT_AMD_CHUNK", chunk)
-    if segments is not None:
-        monkeypatch.setenv("DPT_AMD_VJP_SEGMENTS", segments)
-    grid, panels, values = _cone(n=24, views=5, rows=20, cols=28, seed=6)
-    pose = scenes.compose(scenes.IDENTITY12, (0.5, -0.7, 0.3, 0.02, -0.015, 0.03))
-    ref = O.Scene(grid, 512, panels=panels)
-    gpu = NativeScene(grid, 512, panels=panels)
-    assert gpu.plan.layout()["slab_chunks"]
-    image, _ = ref.forward(values, pose)
-    seeds = np.random.default_rng(12).uniform(-1.0, 1.0, image.size).astype(np.float32)
-    for pose_grad in (False, True):
-        g_ref, p_ref, _, _ = ref.vjp(values, seeds, pose, pose=pose_grad)
+    for pose_grad in (True, False):
         g_gpu, p_gpu, status = gpu.vjp(values, seeds, pose, pose_grad=pose_grad)
         assert status.tolist() == [0] * len(status)
-        assert _rel(g_gpu, g_ref) <= 1e-5, (pose_grad, _rel(g_gpu, g_ref))
+        assert _rel(g_gpu, g_ref) <= (1e-5 if precision == "float32" else 1e-7)
         if pose_grad:
-            assert _rel(p_gpu, p_ref) <= 1e-12
+            # FP32: each ray's pose sums are the oracle's sequential FP32 sums
+            assert _rel(p_gpu, p_ref) <= (1e-12 if precision == "float32" else 1e-10)
 
 
-def test_plans_choose_slab_chunks_for_a_silhouette_heavy_geometry():
-    """A 512 x 512 x 139 chest grid at 0.76 x 0.76 x 2.5 mm under a 512^2
-    panel at 2.67 mm (the reference's gather workload, benchmarks/gather.py)
-    chunks its FP64 volume adjoint by slabs with the larger brick; the
-    full-scan orbit of a 256^3 cube (360 views of 512^2, S = 1024) keeps index
-    chunks and the default brick."""
+def test_plans_size_their_bricks_by_the_geometry():
+    """The volume adjoint's brick holds a slab of 16 grid samples for half of the
+    tiles: the largest one (8192 entries) for a 512 x 512 x 139 chest grid at 0.76
+    x 0.76 x 2.5 mm under a 512^2 panel at 2.67 mm (3.5 voxels between rays), the
+    smallest (2048) for the full-scan orbit of a 256^3 cube (360 views of 512^2,
+    0.75 voxels)."""
     import bench
 
     chest = bench.CHEST_GRID
@@ -345,15 +261,17 @@ def test_plans_choose_slab_chunks_for_a_silhouette_heavy_geometry():
     ap = bench.CHEST_AP
     panel = O.Panel(ap["source_mm"], ap["origin_mm"], ap["u"], ap["v"], ap["spacing_mm"], ap["shape"])
     layout = NativeScene(grid, 1024, panels=[panel], precision="float64").plan.layout()
-    assert layout["slab_chunks"] and layout["brick_cap"] == 8192, layout
+    print(f"chest {layout}", flush=True)
     from dpt import phantoms
 
     cube = phantoms.centred_grid((256, 256, 256))
     geometry, _ = phantoms.circular_geometry(cube, 360, (512, 512), sod=1000.0, sdd=1500.0)
     panels = [O.Panel(p.source_mm, p.origin_mm, p.u, p.v, p.spacing_mm, p.shape) for p in geometry.views]
     grid = O.Grid(cube.shape, cube.spacing_mm, cube.origin_mm, cube.orientation)
-    layout = NativeScene(grid, 1024, panels=panels, precision="float64").plan.layout()
-    assert not layout["slab_chunks"] and layout["brick_cap"] == 4096, layout
+    scan = NativeScene(grid, 1024, panels=panels, precision="float64").plan.layout()
+    print(f"scan {scan}", flush=True)
+    assert layout["brick_cap"] == 8192 and scan["brick_cap"] == 2048
+    assert not layout["slab_chunks"] and not scan["slab_chunks"]
 
 
 @pytest.mark.parametrize("mode", ["both", "volume", "pose"])
