@@ -604,8 +604,8 @@ __device__ __forceinline__ double gather_voxel(const Params &P, const GatherRay 
 // on six, 8.7 on eight; whole calls on two / four / six: 60 views of 64^2 into
 // 16^3 29.8 / 13.4 / 13.3 ms, of 96^2 into 64^3 9.2 / 3.4 / 3.5, 8 views of 200^2
 // into 200^3 3.3 / 2.9 / 2.9, one of 512^2 into 139 x 512 x 512 1.26 / 1.23 /
-// 1.21, a cylindrical one of 32^2 into 32^3 0.46 / 0.47 / 0.50.)  The lanes of surface bricks that fall on an edge line
-// are idle.
+// 1.21, a cylindrical one of 32^2 into 32^3 0.46 / 0.47 / 0.50.)  The lanes of
+// surface bricks that fall on an edge line are idle.
 constexpr int kEdgeVoxels = 16;  // voxels of an edge wave, a quad of lanes each
 
 struct BrickLayout {

@@ -1458,7 +1458,7 @@ __global__ __launch_bounds__(kBlock, 3) void vjp_gauss_kernel(Params P, const T 
 // are linear in the sample index, so the corner sums of the cell's n samples
 // follow from the fractions m at their mean and the variance v = (n^2 - 1) / 12
 // of the index: sum fx fy = n (mx my + v bx by), b the advance per sample, and
-// likewise the triple product (the odd moments vanish).  About 76 VALU
+// likewise the triple product (the odd moments vanish).  About 80 VALU
 // instructions a cell, against 110 a sample (2.5 samples a cell on the full
 // scan) when every sample formed its weights; the sums leave out the FP32
 // rounding of each sample's position (volume gradient of a 4-view full scan
@@ -1489,9 +1489,9 @@ __global__ __launch_bounds__(kBlock, 3) void vjp_gauss_kernel(Params P, const T 
 // Bound by the device atomics of the drain (one request per 64-byte block,
 // 23.6 G/s), the LDS atomics and VALU issue, in turn.  MI355X, before (per
 // sample, joint with the pose) and after (walk + pose launch): 360-view 512^2
-// scan of 256^3 at S = 1024 262 -> 68 + 87 ms; 24 views of 256^2 over 256^3 in
-// bfloat16 24.5 -> 6.2 + 2.4 ms; 60 views of 256^2 over 128^3 (volume only)
-// 7.8 -> 2.4 ms; FP64 24 views of 256^2 over 128^3 18.5 -> 1.0 + 2.6 ms.
+// scan of 256^3 at S = 1024 262 -> 62 + 74 ms; 24 views of 256^2 over 256^3 in
+// bfloat16 24.5 -> 5.7 + 2.2 ms; 60 views of 256^2 over 128^3 (volume only)
+// 7.8 -> 2.0 ms; FP64 24 views of 256^2 over 128^3 18.5 -> 0.9 + 2.2 ms.
 // A ray in sample-index units: coordinate a of sample k is A[a] + k B[a].
 struct WalkRay {
     double A[3], B[3];
@@ -1575,7 +1575,7 @@ __device__ __forceinline__ void walk_drain(const Params &P, const Brick &B, doub
 // GAUSS: the exact cell-Gauss rule; the walk runs in the ray parameter, a step is
 // a piece between crossings, and its two nodes at centre +- radius / sqrt(3)
 // are a run of two samples with index variance radius^2 / 3 (24 views of 256^2
-// over 128^3: joint adjoint 4.15 -> 1.74 + 1.05 ms; two products a corner and
+// over 128^3: joint adjoint 4.15 -> 1.09 + 1.45 ms; two products a corner and
 // node and 6.1e7 device atomics before).
 // FP32 sums keep six waves per SIMD (80 VGPRs, 32 bytes of spills; 90 and five
 // without the bound: full scan 61.9 and 62.9 ms), FP64 ones take four (121; five
@@ -1983,8 +1983,9 @@ __global__ __launch_bounds__(kBlock, (std::is_same<R, float>::value ? 6 : 4)) vo
             __syncthreads();
         }
     }
-    // Rays outside the factor range, or with samples outside the support:
-    // the reference's increments, per sample and corner, by device atomics.
+    // Rays outside the factor range, or whose middle sample (FP64: whose first or
+    // last one) falls outside the support: the reference's increments, per sample
+    // and corner, by device atomics.
     if (scattered) {
         if constexpr (std::is_same<S, float>::value) {
             for (int k = first; k < last; ++k) {
