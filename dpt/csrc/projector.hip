@@ -2382,22 +2382,32 @@ void configure_tiles(Params &P, int vb) {
 // won back: enough samples a ray, few waves for them (6 a sample) or rays so
 // far apart that every lane misses its own cells (`dense` rays per face of a
 // voxel; denser lanes share the L1's lines and issue bounds the march, the pose
-// march first), and no four views in a workgroup within two voxels of each
-// other, whose waves share cells a workgroup per wave tile fetches again.  MI355X, a lane per ray against
-// split: one 512^2 view over 128^3 at S = 1: forward 14 and 36 us, pose adjoint
-// 33 and 81; S = 256: 137 and 103, 157 and 177; over 139 x 512 x 512, S = 64:
-// 109 and 79, 124 and 108; 2000 views of 16^2 over 32^3, S = 128: 131 and 179,
-// 181 and 329.  Over 1458 such points (1 to 2000 views, S 1 to 1024, 32^3 to
-// 256^3) the rule is 2 % off the better of both, split wherever it fits 9 %
-// (forward) and 19 % (pose), a lane per ray 34 % and 31 %.
+// march first).  Four views in a workgroup within two voxels of each other share
+// cells at any density, and a workgroup per wave tile fetches them again: only
+// many samples outweigh that, down to half as many on panels above 24^2 pixels
+// as on smaller ones.  MI355X, a lane per ray against split: one 512^2
+// view over 128^3 at S = 1: forward 14 and 36 us, pose adjoint 33 and 81;
+// S = 256: 137 and 103, 157 and 177; over 139 x 512 x 512, S = 64: 109 and 79,
+// 124 and 108; 2000 views of 16^2 over 32^3, S = 128: 131 and 179, 181 and 329;
+// 24 views of 80^2 at one angle over 128^3, S = 64: 42 and 51, 59 and 85; S =
+// 1000: 267 and 195, 454 and 328.
+// Over 1458 points of views a degree or more apart on a circle, or 2000 of
+// them (1 to 2000 views, S 1 to 1024, 32^3 to 256^3) the rule is 2 % off the
+// better of both, split wherever it fits 9 % (forward) and 19 % (pose), a lane
+// per ray 34 % and 31 %; over 540 of 4 to 32 views at one angle or within 8
+// degrees it is 5 % off (forward) and 2 % (pose), split 7 % and 15 %, a lane per
+// ray 19 % and 20 %.
 bool split_launch(const dpt_plan *p, const Params &P, bool pose) {
     const long long waves = (long long)P.total_tiles * (kBlock / 64);
     if (waves > 8192) return false;
     if (waves <= 512) return true;
-    if (P.samples < (pose ? 48 : 32) || (P.vb == 4 && p->view_gap < 2.0)) return false;
+    if (P.samples < (pose ? 48 : 32)) return false;
+    const bool near = P.vb == 4 && p->view_gap < 2.0;
+    if (waves <= (near && P.rows * P.cols >= 24 * 24 ? 12LL : 6LL) * P.samples) return true;
+    if (near) return false;
     const double side = std::cbrt((double)P.nx * P.ny * P.nz);
     const double rays_per_face = (double)P.vb * P.rows * P.cols / (side * side), dense = pose ? 4.5 : 32.0;
-    return waves <= 6LL * P.samples || rays_per_face <= dense;
+    return rays_per_face <= dense;
 }
 
 // Sample-range segments of the volume adjoint: a launch of few tiles (one view
