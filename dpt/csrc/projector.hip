@@ -1472,19 +1472,24 @@ __global__ __launch_bounds__(kBlock, 3) void vjp_gauss_kernel(Params P, const T 
 // costs no lockstep waste; a slab whose box overflows the brick is halved, and
 // the next one doubled while it fits.
 //
-// Where rays lie more than about three voxels apart (kWalkSparse) a brick holds
+// Where rays lie more than three to four voxels apart (kWalkSparse) a brick holds
 // mostly zeros: its box fills the LDS with a slab of a few samples, and the
 // bounds, barriers and drain of every slab cost more than the few sums they
 // merge.  Such a workgroup adds its corner sums by device atomics at once, two
 // x-adjacent entries a request from a pair of lanes; it is found when a slab of
 // eight samples overflows (asked at sixteen, 30 views of 128^2 over 128^3 ran 6
 // % slower; asked at four, 24 views of 128^2 over 256^3 at S = 64 took 4.3
-// instead of 2.1 ms).  MI355X, bricks and atomics: 24 views over 256^3 at S =
-// 512, panels of 96^2 / 128^2 / 160^2 (0.06 / 0.11 / 0.17 rays a voxel) 8.6 and
-// 4.3 / 9.2 and 7.5 / 12.4 and 11.6 ms, of 192^2 (0.25) 8.5 and 16.4; 60 views
-// of 24^2 over 128^3 3.9 and 0.45 ms; 24 x 256^2 over 512^3 at S = 128 33.7 and
-// 12.6; 2^18 random rays in 256^3 5.8 and 2.2; 2^16 by the exact rule in 128^3
-// 1.51 and 0.49.
+// instead of 2.1 ms).  Bricks pay longer for rays along y and z: their slabs are
+// thin across x no more than the rays allow, and a drain request adds a run of
+// a row, where the entries of rays along x follow one another in pairs anyway.
+// MI355X, bricks and atomics: 24 views over 256^3 at S = 512, panels of 96^2 /
+// 128^2 / 160^2 (0.06 / 0.11 / 0.17 rays a voxel) 8.6 and 4.3 / 9.2 and 7.5 /
+// 12.4 and 11.6 ms, of 192^2 (0.25) 8.5 and 16.4; 60 views of 24^2 over 128^3
+// 3.9 and 0.45 ms; 2^18 random rays in 256^3 5.8 and 2.2; 2^16 by the exact rule
+// in 128^3 1.51 and 0.49.  Over 101 scenes of 20 to 30 views (128 x 40 x 128 to
+// 512^3, 0.06 to 0.2 rays a voxel, S 48 to 1024) the walk takes 0.56 of the time of
+// bricks alone, worst 1.29 (1.7 -> 2.2 ms, 300 x 74 x 225 at S = 1000), with 0.12
+// for every axis 0.60 and 1.54.
 //
 // Bound by the device atomics of the drain (one request per 64-byte block,
 // 23.6 G/s), the LDS atomics and VALU issue, in turn.  MI355X, before (per
@@ -1501,7 +1506,9 @@ constexpr double kWalkBias = 0x1.8p20;         // 1.5 * 2^20: a sum's low word i
 constexpr int kWalkBiasHigh = 0x41380000;      // high word of the bias: the difference is floor(coordinate)
 constexpr int kWalkWidth = 16;                  // grid samples of the first slab
 constexpr int kWalkMaxAxis = 1 << 18;          // largest axis of the biased form
-constexpr float kWalkSparse = 0.12f;           // least rays per grid sample of a slab's cross-section worth a brick
+// Least rays per grid sample of a slab's cross-section worth a brick: rays that
+// advance fastest along x, and others.
+constexpr float kWalkSparseX = 0.12f, kWalkSparse = 0.06f;
 
 // Floor and fraction of coordinate a of sample k (R float: through the bias,
 // 2^-32 resolution; R double: exact).
@@ -1795,7 +1802,8 @@ __global__ __launch_bounds__(kBlock, (std::is_same<R, float>::value ? 6 : 4)) vo
             Brick B{};
             (void)chunk_brick(P, bound_red, blo, bnhi, P.walk_cap, P.nx > 1, B, e);
             const float across = axis == 0 ? (float)e[1] * e[2] : (axis == 1 ? (float)e[0] * e[2] : (float)e[0] * e[1]);
-            const bool sparse = (float)(ray_red[0] + ray_red[1] + ray_red[2] + ray_red[3]) < kWalkSparse * across;
+            const bool sparse = (float)(ray_red[0] + ray_red[1] + ray_red[2] + ray_red[3]) <
+                                (axis == 0 ? kWalkSparseX : kWalkSparse) * across;
             return (bool)__builtin_amdgcn_readfirstlane(sparse);
         };
         bool weighed = false, sparse = false;  // asked once, when a thin slab's box overflows the brick

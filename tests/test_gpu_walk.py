@@ -70,12 +70,13 @@ def test_slabs_that_fit_no_brick_use_device_atomics(precision, monkeypatch):
 @pytest.mark.parametrize("views_per_block", ["1", "2", "4"])
 @pytest.mark.parametrize("samples", [1, 7, 61, 900])
 @pytest.mark.parametrize("precision", ["float32", "float64"])
-def test_sparse_rays_add_by_pairs_of_lanes(samples, precision, views_per_block, monkeypatch):
-    """Rays four voxels apart walk without bricks, the wave as one, until its last
-    ray ends."""
-    print(f"case walk sparse S={samples} {precision} vb={views_per_block}", flush=True)
+@pytest.mark.parametrize("rows,cols", [(16, 15), (9, 10)])
+def test_sparse_rays_add_by_pairs_of_lanes(rows, cols, samples, precision, views_per_block, monkeypatch):
+    """Rays four (along x) and seven voxels apart (along any axis) walk without
+    bricks, the wave as one, until its last ray ends."""
+    print(f"case walk sparse {rows}x{cols} S={samples} {precision} vb={views_per_block}", flush=True)
     monkeypatch.setenv("DPT_AMD_VIEWS_PER_BLOCK", views_per_block)
-    actual, expected = _volume(_blocky(), samples, precision, views=5, rows=16, cols=15)
+    actual, expected = _volume(_blocky(), samples, precision, views=5, rows=rows, cols=cols)
     assert _rel(actual, expected) <= (1e-5 if precision == "float32" else 1e-7)
 
 
